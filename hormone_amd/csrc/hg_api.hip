@@ -216,6 +216,24 @@ extern "C" int hg_create(const hg_desc *desc, hg_ctx **out) {
                        c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
       return fail(HG_ERR_DEVICE);
+    // the FP64 slopes' grid factors; the fast divisions rely on spacings
+    // within 2^+-100 and limiter ratios within 2^+-8 (cell_faces, fslope)
+    for (int a = 0; a < 3; ++a) {
+      const int m = nn[a] + 4;
+      double2 *geo = nullptr;
+      if ((st = dev_alloc(c, sizeof(double2) * 6 * (size_t)m, (void **)&geo))) return fail(st);
+      launch_geo(D.ax[a], geo, c->stream);
+      D.ax[a].geo = geo + 2;
+      const double *x = src[a][0], *xi = src[a][1], *idx = src[a][4];
+      auto in = [](double v, int e) { return v > std::ldexp(1.0, -e) && v < std::ldexp(1.0, e); };
+      bool ok = true;
+      for (int q = 1; q < m - 1; ++q)  // array element q holds cell q-2
+        ok = ok && in(x[q + 1] - x[q], 100) && in(x[q] - x[q - 1], 100) &&
+             in((x[q + 1] - x[q]) / (xi[q] - x[q]), 8) &&
+             in((x[q] - x[q - 1]) / (x[q] - xi[q - 1]), 8) && in(idx[q], 100) &&
+             in(idx[q + 1], 100);
+      D.ax[a].fast = ok;
+    }
     // mixed-precision limiter geometry, indices -2..n+1 per axis
     for (int a = 0; a < 3; ++a) {
       const int m = nn[a] + 4;

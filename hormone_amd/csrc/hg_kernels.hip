@@ -382,6 +382,20 @@ __device__ __forceinline__ void cell_ijk(const Dev &D, long m, int &i, int &j, i
   k = (int)kk;
 }
 
+// the lane's own cell of a loaded tile (zero: 0, see sweep_line)
+template <int DIR, bool MAG>
+__device__ __forceinline__ Cell tile_column(const Dev &D, const Axis &A, int c,
+                                            const double *lds, int zero = 0) {
+  const int bw = blockDim.x >> 6, w = threadIdx.x >> 6, lane = (threadIdx.x & 63) + zero;
+  const int ld = tile_ld(bw), fs = 64 * ld;
+  const int nf = MAG ? NWMAX : WEINT + 1;
+  double f[NWMAX];
+  const double *p = lds + lane * ld + w;
+#pragma unroll
+  for (int k = 0; k < NWMAX; ++k) f[k] = k < nf ? p[k * fs] : 0.0;
+  return finish_cell<DIR, MAG>(D, A, c, f);
+}
+
 template <int DIR, bool MAG, bool EXT = true>
 __device__ __forceinline__ Cell tile_cell(const Dev &D, const Axis &A, long wave0, long base,
                                           int c, bool valid, double *lds) {
@@ -431,11 +445,7 @@ __device__ __forceinline__ Cell tile_cell(const Dev &D, const Axis &A, long wave
     }
   }
   __syncthreads();
-  double f[NWMAX];
-  const double *p = lds + lane * ld + w;
-#pragma unroll
-  for (int k = 0; k < NWMAX; ++k) f[k] = k < nf ? p[k * fs] : 0.0;
-  return finish_cell<DIR, MAG>(D, A, c, f);
+  return tile_column<DIR, MAG>(D, A, c, lds);
 }
 
 // Thread t's row of the tile on the way out: true with its element index m
@@ -510,9 +520,10 @@ __device__ __forceinline__ double dn1(double x) {
 
 // Limited slopes of a cell (interpolation.f90, loop c = -1 .. n) and the
 // e_int guard (interpolation.f90:143-163).  qv, ql, qr: d e m1 m2 m3 b1 b2 b3
-// eint of the cell and of its left and right neighbours.  SH: divisions by
-// the grid denominators shared between the variables (qdiv).
-template <bool MAG, int LIM, bool SH>
+// eint of the cell and of its left and right neighbours.  Plain divisions: the
+// form a wavefront takes when the fast one (cell_faces) met an operand of
+// extreme exponent.
+template <bool MAG, int LIM>
 __device__ __forceinline__ void cell_slopes(const double qv[9], const double ql[9],
                                             const double qr[9], double xm, double x0, double xp,
                                             double xim, double xi0, double ida, double idb,
@@ -521,8 +532,8 @@ __device__ __forceinline__ void cell_slopes(const double qv[9], const double ql[
   // grid factors and denominators shared by every variable of the cell
   const double dxp = xp - x0;
   const double cf = dxp / (xi0 - x0), cb = (x0 - xm) / (x0 - xim);
-  const auto Dm = mkden<SH>(LIM == LIM_MINMOD ? ida + idb : x0 - xm);
-  const auto Dp = mkden<SH>(dxp);
+  const auto Dm = mkden<false>(LIM == LIM_MINMOD ? ida + idb : x0 - xm);
+  const auto Dp = mkden<false>(dxp);
   double fl[8], fr[8];
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
@@ -537,6 +548,7 @@ __device__ __forceinline__ void cell_slopes(const double qv[9], const double ql[
     S[s] = du;
     fl[s] = qv[s] - hl * du;
     fr[s] = qv[s] + hr * du;
+    fence();
   }
   double eintl = fl[1] - 0.5 * (fl[2] * fl[2] + fl[3] * fl[3] + fl[4] * fl[4]) / fl[0];
   double eintr = fr[1] - 0.5 * (fr[2] * fr[2] + fr[3] * fr[3] + fr[4] * fr[4]) / fr[0];
@@ -556,9 +568,9 @@ __device__ __forceinline__ void cell_slopes(const double qv[9], const double ql[
 // the lane's cell (left: L = d e m1 m2 m3 b1 b2 b3 phi, slopes S) and the
 // right neighbour (R, RS) -- numflux.f90 with the cyclic rotation normal a =
 // DIR, then b, c (numflux.f90:73-93,246-266,419-439).  Returns the face
-// densities and internal energies for the positivity check.  SH: divisions
-// by dl, dr and the HLLD denominators shared between numerators (qdiv).
-template <int DIR, bool MAG, bool SH>
+// densities and internal energies for the positivity check.  Plain divisions
+// and square roots, as cell_slopes (the fast form is face_fast).
+template <int DIR, bool MAG>
 __device__ __forceinline__ void face_flux(const double L[9], const double S[8],
                                           const double R_[9], const double RS[8], double dx1,
                                           double dx2, double gam, double ch, double t[9],
@@ -568,13 +580,16 @@ __device__ __forceinline__ void face_flux(const double L[9], const double S[8],
   const double dr = R_[0] - dx2 * RS[0];
   const double el = L[1] + dx1 * S[1];
   const double er = R_[1] - dx2 * RS[1];
-  const auto Dl = mkden<SH>(dl), Dr = mkden<SH>(dr);  // every division by dl, dr below
+  const auto Dl = mkden<false>(dl), Dr = mkden<false>(dr);  // every division by dl, dr below
   const double v1l = qdiv(Dl, L[2 + a_] + dx1 * S[2 + a_]);
   const double v1r = qdiv(Dr, R_[2 + a_] - dx2 * RS[2 + a_]);
+  fence();
   const double v2l = qdiv(Dl, L[2 + b_] + dx1 * S[2 + b_]);
   const double v2r = qdiv(Dr, R_[2 + b_] - dx2 * RS[2 + b_]);
+  fence();
   const double v3l = qdiv(Dl, L[2 + c_] + dx1 * S[2 + c_]);
   const double v3r = qdiv(Dr, R_[2 + c_] - dx2 * RS[2 + c_]);
+  fence();
   double b1l = 0, b1r = 0, b2l = 0, b2r = 0, b3l = 0, b3r = 0, phil = 0, phir = 0;
   if (MAG) {
     b1l = L[5 + a_] + dx1 * S[5 + a_];
@@ -597,16 +612,21 @@ __device__ __forceinline__ void face_flux(const double L[9], const double S[8],
   // positive cs2 and is omitted.
   double ptl = (gam - 1.0) * eil;
   double ptr = (gam - 1.0) * eir;
+  fence();
   const double csl = sqrt(qdiv(Dl, gam * ptl));
+  fence();
   const double csr = sqrt(qdiv(Dr, gam * ptr));
+  fence();
   if (MAG) {
     ptl = ptl + 0.5 * (b1l * b1l + b2l * b2l + b3l * b3l);
     ptr = ptr + 0.5 * (b1r * b1r + b2r * b2r + b3r * b3r);
   }
   const double cfl = get_cf_d(Dl, csl, b1l, b2l, b3l);
+  fence();
   const double cfr = get_cf_d(Dr, csr, b1r, b2r, b3r);
-  hlld_d<SH>(t, cfl, cfr, v1l, v1r, v2l, v2r, v3l, v3r, dl, dr, el, er, ptl, ptr, b1l, b1r,
-             b2l, b2r, b3l, b3r, phil, phir, ch);
+  fence();
+  hlld(t, cfl, cfr, v1l, v1r, v2l, v2r, v3l, v3r, dl, dr, el, er, ptl, ptr, b1l, b1r, b2l, b2r,
+       b3l, b3r, phil, phir, ch);
 }
 
 // Mass flux of the face c+1/2 for the species pass (compswitch 2): FM[d]
@@ -647,6 +667,122 @@ __device__ __forceinline__ void boundary_flux(const Axis &A, int c, double t[9])
   t[8] = F[8];
 }
 
+// conserved values and eint the slopes are taken of
+template <bool MAG>
+__device__ __forceinline__ void slope_values(const Cell &q, double qv[9]) {
+  qv[0] = q.d;
+  qv[1] = q.e;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    qv[2 + a] = q.d * q.v[a];
+    qv[5 + a] = MAG ? q.b[a] : 0.0;
+  }
+  qv[8] = q.eint;
+}
+
+// The grid factors of cell c's slopes (k_geo's table).
+template <int LIM>
+__device__ __forceinline__ Geo load_geo(const Axis &A, int c) {
+  const double2 *g = gptr(A.geo) + c;
+  const int m = A.n + 4;
+  Geo G;
+  const double2 h = g[0];
+  G.hl = h.x;
+  G.hr = h.y;
+  if constexpr (LIM == LIM_MINMOD) {
+    const double2 i = g[4 * m], d = g[5 * m];
+    G.ida = i.x;
+    G.idb = i.y;
+    G.Dab = Den64{d.x, d.y};
+  } else if constexpr (LIM == LIM_MC) {
+    const double2 p = g[m], d = g[2 * m], f = g[3 * m];
+    G.Dp = Den64{p.x, p.y};
+    G.Dm = Den64{d.x, d.y};
+    G.cf = f.x;
+    G.cb = f.y;
+  }
+  return G;
+}
+
+// Flux t of the face c+1/2 of every lane of a wavefront from the lanes' cells
+// (checked fast form).  True, for the whole wavefront, when one of its
+// faces -1 .. n-1 depends on a value out of the fast form's range.
+template <int DIR, bool MAG, int LIM>
+__device__ __forceinline__ bool line_faces(const Axis &A, const Cell &q, int c, int cc, int lane,
+                                           double gam, const Den64 &Dch, double t[9],
+                                           double fe[4]) {
+  const int n = A.n;
+  double qv[9], ql[9], qr[9];
+  slope_values<MAG>(q, qv);
+  unsigned long long bad = __builtin_amdgcn_ballot_w64(odd_cell<MAG>(qv));
+  if (LIM != LIM_FLAT) {
+#pragma unroll
+    for (int s = 0; s < 9; ++s) {
+      ql[s] = up1(qv[s]);
+      qr[s] = dn1(qv[s]);
+    }
+  }
+  const Geo G = load_geo<LIM>(A, cc);
+  double FL[8], FR[8], R_[8];
+  Den64 DL, DR, Dr;
+  Chk kc;
+  cell_faces<MAG, LIM>(qv, ql, qr, G, FL, FR, DL, DR, kc);
+  // lane 0 has no left neighbour; a slope of cell n also relies on the tests
+  // of cell n+1 (fslope)
+  bad |= __builtin_amdgcn_ballot_w64(c >= -1 && lane >= 1 && kc.bad());
+  // the right cell's left face state from lane+1
+#pragma unroll
+  for (int s = 0; s < 8; ++s) R_[s] = (!MAG && s >= 5) ? 0.0 : dn1(FL[s]);
+  Dr.b = R_[0];
+  Dr.r = dn1(DL.r);
+  const double phil = MAG ? q.phi + 0.0 : 0.0;
+  const double phir = MAG ? dn1(phil) : 0.0;
+  Chk kf;
+  face_fast<DIR, MAG>(FR, R_, phil, phir, DR, Dr, gam, Dch, t, fe, kf);
+  bad |= __builtin_amdgcn_ballot_w64(c >= -1 && c <= n - 1 && lane >= 1 && lane <= 61 && kf.bad());
+  return bad != 0 || !A.fast;
+}
+
+// The same in plain divisions and square roots.
+template <int DIR, bool MAG, int LIM>
+__device__ __forceinline__ void line_faces_plain(const Axis &A, const Cell &q, int cc, double gam,
+                                                 double ch, double t[9], double fe[4]) {
+  const int n = A.n;
+  double qv[9];
+  slope_values<MAG>(q, qv);
+  // ---- slopes of cell c (interpolation.f90, loop c = -1 .. n) -----------
+  double S[8];  // dd de dm1 dm2 dm3 db1 db2 db3 (dphi is always 0)
+  if (LIM == LIM_FLAT) {
+#pragma unroll
+    for (int s = 0; s < 8; ++s) S[s] = 0.0;
+  } else {
+    double ql[9], qr[9];
+#pragma unroll
+    for (int s = 0; s < 9; ++s) {
+      ql[s] = up1(qv[s]);
+      qr[s] = dn1(qv[s]);
+    }
+    const int cl = cc > -1 ? cc : -1, cr = cc < n ? cc : n;  // keep indices in range
+    const double xm = gptr(A.x)[cl - 1], x0 = gptr(A.x)[cl], xp = gptr(A.x)[cr + 1];
+    const double xim = gptr(A.xi)[cl - 1], xi0 = gptr(A.xi)[cl];
+    const double ida = gptr(A.idx)[cl], idb = gptr(A.idx)[cr + 1];
+    cell_slopes<MAG, LIM>(qv, ql, qr, xm, x0, xp, xim, xi0, ida, idb, S);
+  }
+  // ---- face c+1/2 (numflux.f90, faces c = -1 .. n-1) ---------------------
+  // right cell's primitives and slopes from lane+1
+  double L[9], R_[9], RS[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) L[s] = qv[s];
+  L[8] = q.phi;
+#pragma unroll
+  for (int s = 0; s < 9; ++s) R_[s] = (!MAG && s >= 5) ? 0.0 : dn1(L[s]);
+#pragma unroll
+  for (int s = 0; s < 8; ++s) RS[s] = (!MAG && s >= 5) ? 0.0 : dn1(S[s]);
+  const int cf_ = cc < n - 1 ? (cc > -1 ? cc : -1) : n - 1;  // clamp face index
+  const double dx1 = gptr(A.xi)[cf_] - gptr(A.x)[cf_], dx2 = gptr(A.x)[cf_ + 1] - gptr(A.xi)[cf_];
+  face_flux<DIR, MAG>(L, S, R_, RS, dx1, dx2, gam, ch, t, fe);
+}
+
 // RK update of the cells a fused sweep has just finished (defined with the RK
 // kernels below)
 template <int DIR, bool MAG, bool TILE>
@@ -674,47 +810,20 @@ __device__ __forceinline__ void sweep_line(const Dev &D, long wave, int lane, in
   const Cell q = TILE ? tile_cell<DIR, MAG, EXT>(D, A, wave0, base, c, valid, lds)
                       : load_cell<DIR, MAG, EXT>(D, A, base, line, c);
   if (FUSED && !TILE) park_cell<MAG>(lds, q);
-  // d e m1 m2 m3 b1 b2 b3 and eint (slopes) / phi (face) of the cell
-  const double qv[9] = {q.d, q.e, q.d * q.v[0], q.d * q.v[1], q.d * q.v[2],
-                        q.b[0], q.b[1], q.b[2], q.eint};
-
-  // ---- slopes of cell c (interpolation.f90, loop c = -1 .. n) -----------
-  double S[8];  // dd de dm1 dm2 dm3 db1 db2 db3 (dphi is always 0)
   const int cc = c < -2 ? -2 : (c > n + 1 ? n + 1 : c);
-  if (LIM == LIM_FLAT) {
-#pragma unroll
-    for (int s = 0; s < 8; ++s) S[s] = 0.0;
-  } else {
-    double ql[9], qr[9];
-#pragma unroll
-    for (int s = 0; s < 9; ++s) {
-      ql[s] = up1(qv[s]);
-      qr[s] = dn1(qv[s]);
-    }
-    const int cl = cc > -1 ? cc : -1, cr = cc < n ? cc : n;  // keep indices in range
-    const double xm = gptr(A.x)[cl - 1], x0 = gptr(A.x)[cl], xp = gptr(A.x)[cr + 1];
-    const double xim = gptr(A.xi)[cl - 1], xi0 = gptr(A.xi)[cl];
-    const double ida = gptr(A.idx)[cl], idb = gptr(A.idx)[cr + 1];
-    cell_slopes<MAG, LIM, true>(qv, ql, qr, xm, x0, xp, xim, xi0, ida, idb, S);
-  }
-
-  // ---- face c+1/2 (numflux.f90, faces c = -1 .. n-1) ---------------------
-  // right cell's primitives and slopes from lane+1
-  double L[9], R_[9];
-#pragma unroll
-  for (int s = 0; s < 8; ++s) L[s] = qv[s];
-  L[8] = q.phi;
-#pragma unroll
-  for (int s = 0; s < 9; ++s) R_[s] = (!MAG && s >= 5) ? 0.0 : dn1(L[s]);
-  double RS[8];
-#pragma unroll
-  for (int s = 0; s < 8; ++s) RS[s] = (!MAG && s >= 5) ? 0.0 : dn1(S[s]);
-
-  const int cf_ = cc < n - 1 ? (cc > -1 ? cc : -1) : n - 1;  // clamp face index
-  const double dx1 = gptr(A.xi)[cf_] - gptr(A.x)[cf_], dx2 = gptr(A.x)[cf_ + 1] - gptr(A.xi)[cf_];
-  const double gam = D.gamma, ch = gptr(D.sc)->ch;
+  const double gam = D.gamma;
+  const Den64 Dch{gptr(D.sc)->ch, gptr(D.sc)->chr};
   double t[9], fe[4];
-  face_flux<DIR, MAG, true>(L, S, R_, RS, dx1, dx2, gam, ch, t, fe);
+  const bool odd = line_faces<DIR, MAG, LIM>(A, q, c, cc, lane, gam, Dch, t, fe);
+  if (odd) {  // the whole wavefront: its cells again, in plain divisions
+    int c2 = c;
+    asm volatile("" : "+v"(c2));  // read again, not kept from above
+    Cell q2;
+    if (TILE) q2 = tile_column<DIR, MAG>(D, A, c2, lds, c2 - c);
+    else q2 = load_cell<DIR, MAG, EXT>(D, A, base, line, c2);
+    line_faces_plain<DIR, MAG, LIM>(A, q2, c2 < -2 ? -2 : (c2 > n + 1 ? n + 1 : c2), gam,
+                                    gptr(D.sc)->ch, t, fe);
+  }
   const bool fxb = EXT && A.ext && flux_face(A, c);
   if (fxb) boundary_flux<DIR>(A, c, t);
   // faces between lanes l and l+1 have valid slopes on both sides for l = 1..61
@@ -1667,6 +1776,7 @@ __device__ __forceinline__ void cfl_final(const Dev &D) {
     if (sc->endstyle == 1) dt = mn2(dt, t_end - time);
     sc->dt = dt;
     sc->ch = b;
+    sc->chr = fden(b).r;
   }
 }
 
@@ -1882,6 +1992,29 @@ __global__ __launch_bounds__(256) void k_bstep_end_cfl(Batch B) {
   cfl_final(D);
 }
 
+// The slopes' grid factors of one axis, evaluated once per context from the
+// operands the plain path reads (the same bits): rows of n+4 pairs, cells -2
+// .. n+1: (hl, hr), (dxp, 1/dxp), (dxm, 1/dxm), (cf, cb), (ida, idb), (ida +
+// idb, its reciprocal).  Cells past a slope's range (-2, n+1) take their
+// neighbour's.  In the sweep they took two divisions and two reciprocals per
+// lane.
+__global__ void k_geo(Axis A, double2 *geo) {
+  const int m = A.n + 4;
+  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < m; q += gridDim.x * blockDim.x) {
+    const int c = q < 1 ? -1 : (q > m - 2 ? A.n : q - 2);
+    const double xm = A.x[c - 1], x0 = A.x[c], xp = A.x[c + 1];
+    const double xim = A.xi[c - 1], xi0 = A.xi[c];
+    const double ida = A.idx[c], idb = A.idx[c + 1];
+    const double dxp = xp - x0, dxm = x0 - xm, dab = ida + idb;
+    geo[q] = make_double2(x0 - xim, xi0 - x0);
+    geo[m + q] = make_double2(dxp, fden(dxp).r);
+    geo[2 * m + q] = make_double2(dxm, fden(dxm).r);
+    geo[3 * m + q] = make_double2(dxp / (xi0 - x0), dxm / (x0 - xim));
+    geo[4 * m + q] = make_double2(ida, idb);
+    geo[5 * m + q] = make_double2(dab, fden(dab).r);
+  }
+}
+
 __global__ void k_clear_error(Scalars *sc) { sc->err = NOERR; }
 
 // dt, ch and the error status of a finished CFL reduction into a caller's
@@ -1895,6 +2028,7 @@ __global__ void k_timestep_out(const Scalars *sc, double *out) {
 __global__ void k_set_step(Scalars *sc, double dt, double ch) {
   sc->dt = dt;
   sc->ch = ch;
+  sc->chr = fden(ch).r;
   sc->stop = STOP_NONE;
 }
 
@@ -1921,47 +2055,103 @@ __global__ __launch_bounds__(256) void k_phidamp(Dev D, double factor) {
 }
 
 // ---- known-answer evaluation of the device arithmetic -----------------------
-// SH: the forms the sweep runs, with divisions by a shared denominator (qdiv)
-template <bool SH>
+// FAST: the forms the sweep runs (checked fast divisions and square roots,
+// plain ones for a record out of their range)
+template <bool FAST>
 __device__ void kat_one(int which, long t, const double *in, double *out) {
   if (which == 0) {  // hlldflux: 25 inputs (hlldflux.f90:19-21 order), 9 outputs
     const double *a = in + 25 * t;
     double f[9];
-    hlld_d<SH>(f, a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9], a[10], a[11],
-               a[12], a[13], a[14], a[15], a[16], a[17], a[18], a[19], a[20], a[21], a[22]);
+    Chk k;
+    if (FAST)
+      hlld_fast<true>(f, a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9], a[10], a[11],
+                      a[12], a[13], a[14], a[15], a[16], a[17], a[18], a[19], a[20], a[21],
+                      fden(a[22]), k);
+    if (!FAST || k.bad())
+      hlld(f, a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9], a[10], a[11], a[12],
+           a[13], a[14], a[15], a[16], a[17], a[18], a[19], a[20], a[21], a[22]);
     for (int s = 0; s < 9; ++s) out[9 * t + s] = f[s];
   } else if (which == 1) {  // get_cf: d cs b1 b2 b3
     const double *a = in + 5 * t;
-    out[t] = get_cf_d(mkden<SH>(a[0]), a[1], a[2], a[3], a[4]);
-  } else if (which == 2) {  // modified_mc: u0 u1 u2 xm x0 xp xim xi0
-    const double *a = in + 8 * t;
-    const double xm = a[3], x0 = a[4], xp = a[5], xim = a[6], xi0 = a[7];
-    const double dxp = xp - x0;
-    const double cf = dxp / (xi0 - x0), cb = (x0 - xm) / (x0 - xim);
-    out[t] = modified_mc_d(a[0], a[1], a[2], dxp, cf, cb, mkden<SH>(x0 - xm), mkden<SH>(dxp));
-  } else if (which == 3) {  // minmod: u0 u1 u2 dxa dxb
-    const double *a = in + 5 * t;
-    out[t] = minmod_d(a[0], a[1], a[2], a[3], a[4], mkden<SH>(a[3] + a[4]));
+    Chk k;
+    double c = 0.0;
+    if (FAST) {
+      k.pos(a[0]);
+      c = fast_cf(fden(a[0]), a[1], a[2], a[3], a[4], k);
+    }
+    if (!FAST || k.bad()) c = get_cf(a[0], a[1], a[2], a[3], a[4]);
+    out[t] = c;
+  } else if (which == 2 || which == 3) {
+    // modified_mc: u0 u1 u2 xm x0 xp xim xi0; minmod: u0 u1 u2 dxa dxb
+    const double *a = in + (which == 2 ? 8 : 5) * t;
+    double r = 0.0;
+    bool bad = !FAST;
+    if (FAST) {
+      Geo G;
+      Chk k;
+      if (which == 2) {
+        G.Dm = fden(a[4] - a[3]);
+        G.Dp = fden(a[5] - a[4]);
+        G.cf = (a[5] - a[4]) / (a[7] - a[4]);
+        G.cb = (a[4] - a[3]) / (a[4] - a[6]);
+        r = fslope<LIM_MC>(a[0], a[1], a[2], G, k);
+        k.num((a[2] - a[1]) * G.Dp.b);  // in the sweep the right neighbour's test
+        k.pos(G.Dm.b);
+        k.pos(G.Dp.b);
+      } else {
+        G.ida = a[3];
+        G.idb = a[4];
+        G.Dab = fden(a[3] + a[4]);
+        r = fslope<LIM_MINMOD>(a[0], a[1], a[2], G, k);
+        k.pos(G.Dab.b);
+      }
+      // the sweep's slope may have a zero of the other sign: as q + h*S
+      // (with q = 0) shows it
+      bad = k.bad() || r == 0.0;
+      for (int s = 0; s < 3; ++s) bad |= __builtin_amdgcn_class(a[s], 0x227);
+    }
+    if (bad)
+      r = which == 2 ? modified_mc(a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7])
+                     : minmod(a[0], a[1], a[2], a[3], a[4]);
+    out[t] = r;
   } else if (which == 4) {  // division and square root: a b -> a/b, sqrt(a)
     const double *a = in + 2 * t;
     out[2 * t] = a[0] / a[1];
     out[2 * t + 1] = sqrt(a[0]);
   } else if (which == 5) {  // division by a shared denominator: b a0 a1 a2 a3 -> ai/b
     const double *a = in + 5 * t;
-    const Den64 Db = mkden<true>(a[0]);
-    for (int s = 0; s < 4; ++s) out[4 * t + s] = qdiv(Db, a[1 + s]);
+    const Den64 Db = fden(a[0]);
+    for (int s = 0; s < 4; ++s) {
+      if (FAST) {
+        Chk k;
+        k.pos(a[0]);
+        k.num(a[1 + s]);
+        out[4 * t + s] = k.bad() ? a[1 + s] / a[0] : fdiv_(Db, a[1 + s]);
+      } else {
+        out[4 * t + s] = qdiv(Db, a[1 + s]);
+      }
+    }
   } else if (which == 6) {  // eos_p_cs as the face states use it: d eint gamma -> p cs
     const double *a = in + 3 * t;
     const double p = (a[2] - 1.0) * a[1];
     out[2 * t] = p;
-    out[2 * t + 1] = sqrt(qdiv(mkden<SH>(a[0]), a[2] * p));
+    double c = 0.0;
+    Chk k;
+    if (FAST) {
+      const double cs2 = fdiv_(fden(a[0]), a[2] * p);
+      k.pos(a[0]);
+      k.pos(cs2);
+      c = fsqrt(cs2);
+    }
+    if (!FAST || k.bad()) c = sqrt(a[2] * p / a[0]);
+    out[2 * t + 1] = c;
   } else if (which == 7) {  // get_eint: etot d v1 v2 v3 b1 b2 b3 mag_on -> eint
     const double *a = in + 9 * t;
     out[t] = get_eint(a[8] > 0.5, a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7]);
   }
 }
 
-// which 0..7 as hg_kat; + 16: the sweep's shared-denominator form
+// which 0..7 as hg_kat; + 16: the form the sweep runs
 __global__ void k_kat(int which, int n, const double *in, double *out) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
@@ -2021,6 +2211,10 @@ size_t sweep_tile_bytes(const Dev &D, int bw) {
 void launch_pressure(const Dev &D, hipStream_t s) {
   if (D.mag) k_pressure<true><<<nblk(D.ncell, 256), 256, 0, s>>>(D);
   else k_pressure<false><<<nblk(D.ncell, 256), 256, 0, s>>>(D);
+}
+
+void launch_geo(const Axis &A, double2 *geo, hipStream_t s) {
+  k_geo<<<nblk(A.n + 4, 256), 256, 0, s>>>(A, geo);
 }
 
 void launch_clear_error(const Dev &D, hipStream_t s) { k_clear_error<<<1, 1, 0, s>>>(D.sc); }

@@ -39,7 +39,7 @@ enum { STOP_NONE = 0, STOP_END = 1, STOP_OUTPUT = 2, STOP_MAXSTEPS = 3, STOP_ERR
 // Device-resident scalars of one context: the hydro step inputs (dt, ch),
 // the CFL reduction results and the main-loop clock of hormone.f90:124-179.
 struct Scalars {
-  double dt, ch;
+  double dt, ch, chr;  // chr: the refined reciprocal of ch (mkden)
   double dtimin, cfmax;
   double time, t_out, t_end, dt_out;
   long long tn, tnlim, tn_out, steps_left;
@@ -55,6 +55,11 @@ struct Axis {
   // idx(i)*idx(i+1)/(idx(i)+idx(i+1))
   const double4 *limg;
   const double *mmw;
+  // FP64 path: the slopes' grid factors (k_geo), element 0 of each row the
+  // interior cell 0; fast: every one of them lies in the range the checked
+  // fast divisions are exact for
+  const double2 *geo;
+  int fast;
   int n;
   unsigned nlines;   // lines along this axis (ncell / n)
   unsigned nsub;     // lines laid end to end in one sweep sequence (lane_cell)
@@ -176,6 +181,7 @@ void launch_bstep_end_cfl(const Batch &B, hipStream_t s);  // per box: step_end,
 void runge_coeff(int stage, int rktype, double *faco, double *fact, double *facn);
 
 void launch_pressure(const Dev &D, hipStream_t s);
+void launch_geo(const Axis &A, double2 *geo, hipStream_t s);  // fills A's geo table
 void launch_clear_error(const Dev &D, hipStream_t s);
 void launch_timestep_out(const Dev &D, double *out, hipStream_t s);  // dt, ch, status
 void launch_set_step(const Dev &D, double dt, double ch, hipStream_t s);

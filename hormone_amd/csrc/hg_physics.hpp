@@ -82,6 +82,12 @@ template <class R> __device__ __forceinline__ R qdiv(const DenX<R> &D, R a) {
   return fdiv(a, D.b);
 }
 
+// A point no instruction is moved across: between the parts of a long straight
+// block it bounds the values in flight (the tests of the fast form would be
+// put off to its end, the plain form's divisions all interleaved: 30 to 70
+// spilled registers).
+__device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
+
 enum { LIM_FLAT = 0, LIM_MINMOD = 1, LIM_MC = 2 };
 
 // fluxlimiter.f90:40-56 (generalised minmod); dx = idx(i:i+1)
@@ -151,12 +157,12 @@ __device__ __forceinline__ R get_cf(R d, R cs, R b1, R b2, R b3) {
 
 // hlldflux + fstar, hlldflux.f90:19-179, without the radiation component
 // (erl = err = 0 on this path; its flux only feeds irad).  f[0..8] are
-// tmpflux(1..9).  SH: FP64 divisions by shared denominators (qdiv).
-template <bool SH, class R>
-__device__ __forceinline__ void hlld_d(R f[9], R cfl, R cfr, R v1l, R v1r, R v2l, R v2r,
-                                       R v3l, R v3r, R dl, R dr, R el, R er, R ptl,
-                                       R ptr, R b1l, R b1r, R b2l, R b2r, R b3l, R b3r,
-                                       R phil, R phir, R ch) {
+// tmpflux(1..9).
+template <class R>
+__device__ __forceinline__ void hlld(R f[9], R cfl, R cfr, R v1l, R v1r, R v2l, R v2r,
+                                     R v3l, R v3r, R dl, R dr, R el, R er, R ptl,
+                                     R ptr, R b1l, R b1r, R b2l, R b2r, R b3l, R b3r,
+                                     R phil, R phir, R ch) {
   const R h = R(0.5);
   R b1 = h * ((b1l + b1r) - fdiv(phir - phil, ch));
   R phi = h * ((phil + phir) - (b1r - b1l) * ch);
@@ -165,52 +171,75 @@ __device__ __forceinline__ void hlld_d(R f[9], R cfl, R cfr, R v1l, R v1r, R v2l
   R sr = mx3(v1r + cfr, v1l + cfl, R(0));
 
   R slv = sl - v1l, srv = sr - v1r;
-  const auto Dden = mkden<SH>(srv * dr - slv * dl);
+  const auto Dden = mkden<false>(srv * dr - slv * dl);
   R sm = qdiv(Dden, srv * dr * v1r - slv * dl * v1l - ptr + ptl);
+  fence();
   R pta = qdiv(Dden, srv * dr * ptl - slv * dl * ptr + dl * dr * srv * slv * (v1r - v1l));
+  fence();
 
   R slm = sl - sm, srm = sr - sm;
-  const auto Dslm = mkden<SH>(slm), Dsrm = mkden<SH>(srm);
+  const auto Dslm = mkden<false>(slm), Dsrm = mkden<false>(srm);
   R dla = qdiv(Dslm, dl * slv);
+  fence();
   R dra = qdiv(Dsrm, dr * srv);
+  fence();
 
   R sqla = rsqrt_(dla), sqra = rsqrt_(dra);
+  fence();
   R sla = sm - fdiv(abs_(b1), sqla);
+  fence();
   R sra = sm + fdiv(abs_(b1), sqra);
+  fence();
 
   R b1b1 = b1 * b1;
-  const auto Dl = mkden<SH>(dl * slv * slm - b1b1);
-  const auto Dr = mkden<SH>(dr * srv * srm - b1b1);
+  const auto Dl = mkden<false>(dl * slv * slm - b1b1);
+  const auto Dr = mkden<false>(dr * srv * srm - b1b1);
   R v2la = v2l - qdiv(Dl, b1 * b2l * (sm - v1l));
+  fence();
   R v2ra = v2r - qdiv(Dr, b1 * b2r * (sm - v1r));
+  fence();
   R v3la = v3l - qdiv(Dl, b1 * b3l * (sm - v1l));
+  fence();
   R v3ra = v3r - qdiv(Dr, b1 * b3r * (sm - v1r));
+  fence();
 
   R numl = dl * slv * slv - b1b1;
   R numr = dr * srv * srv - b1b1;
   R b2la = qdiv(Dl, b2l * numl);
+  fence();
   R b2ra = qdiv(Dr, b2r * numr);
+  fence();
   R b3la = qdiv(Dl, b3l * numl);
+  fence();
   R b3ra = qdiv(Dr, b3r * numr);
+  fence();
 
   R ela = qdiv(Dslm, slv * el - ptl * v1l + pta * sm +
                          b1 * ((v1l * b1 + v2l * b2l + v3l * b3l) -
                                (sm * b1 + v2la * b2la + v3la * b3la)));
+  fence();
   R era = qdiv(Dsrm, srv * er - ptr * v1r + pta * sm +
                          b1 * ((v1r * b1 + v2r * b2r + v3r * b3r) -
                                (sm * b1 + v2ra * b2ra + v3ra * b3ra)));
+  fence();
 
   R sb1 = sgn(R(1), b1);
-  const auto Dsqs = mkden<SH>(sqla + sqra);
+  const auto Dsqs = mkden<false>(sqla + sqra);
   R v2aa = qdiv(Dsqs, sqla * v2la + sqra * v2ra + (b2ra - b2la) * sb1);
+  fence();
   R v3aa = qdiv(Dsqs, sqla * v3la + sqra * v3ra + (b3ra - b3la) * sb1);
+  fence();
   R sqp = rsqrt_(dla * dra);
+  fence();
   R b2aa = qdiv(Dsqs, sqla * b2ra + sqra * b2la + sqp * (v2ra - v2la) * sb1);
+  fence();
   R b3aa = qdiv(Dsqs, sqla * b3ra + sqra * b3la + sqp * (v3ra - v3la) * sb1);
+  fence();
 
   R vbaa = v2aa * b2aa + v3aa * b3aa;
   R eraa = era + sb1 * sqra * ((v2ra * b2ra + v3ra * b3ra) - vbaa);
   R elaa = ela - sb1 * sqla * ((v2la * b2la + v3la * b3la) - vbaa);
+  fence();
 
   R signsm = sgn(h, sm);
   R sortsla = h + sgn(h, sla);
@@ -220,8 +249,10 @@ __device__ __forceinline__ void hlld_d(R f[9], R cfl, R cfr, R v1l, R v1r, R v2l
   R d_ = (h + signsm) * dla + (h - signsm) * dra;
   R v2_ = sortsla * v2la + sortslr * v2aa + sortsra * v2ra;
   R v3_ = sortsla * v3la + sortslr * v3aa + sortsra * v3ra;
+  fence();
   R b2_ = sortsla * b2la + sortslr * b2aa + sortsra * b2ra;
   R b3_ = sortsla * b3la + sortslr * b3aa + sortsra * b3ra;
+  fence();
   R e_ = sortsla * ela + (h - sgn(h, sla * sm)) * elaa + (h + sgn(h, -sm * sra)) * eraa +
          (h - sgn(h, sra)) * era;
 
@@ -237,13 +268,392 @@ __device__ __forceinline__ void hlld_d(R f[9], R cfl, R cfr, R v1l, R v1r, R v2l
   f[7] = b3_ * sm - b1 * v3_;
   f[8] = ch * ch * b1;
 }
-template <class R>
-__device__ __forceinline__ void hlld(R f[9], R cfl, R cfr, R v1l, R v1r, R v2l, R v2r,
-                                     R v3l, R v3r, R dl, R dr, R el, R er, R ptl,
-                                     R ptr, R b1l, R b1r, R b2l, R b2r, R b3l, R b3r,
-                                     R phil, R phir, R ch) {
-  hlld_d<false>(f, cfl, cfr, v1l, v1r, v2l, v2r, v3l, v3r, dl, dr, el, er, ptl, ptr, b1l, b1r,
-                b2l, b2r, b3l, b3r, phil, phir, ch);
+// ---- checked fast arithmetic (the FP64 sweeps) --------------------------------
+// The compiler's FP64 division and square root spend about half of their
+// instructions on scaling operands of extreme exponent (v_div_scale,
+// v_ldexp) and on special results.  The sweep runs them without: fdiv is the
+// same Newton sequence on unscaled operands (4 instructions and a reciprocal
+// shared by every division by that denominator), fsqrt the same coupled
+// iteration.  Where nothing would have been scaled they give the same bits.
+// Whether that held is recorded, not branched on: every divisor, dividend
+// and radicand goes into a Chk, and a wavefront in which one was out of range
+// computes its cells again with plain divisions and square roots
+// (cell_slopes, face_flux).  One test per face instead of a branch per
+// division leaves the compiler one straight block to schedule.  The y and z
+// sweeps are bound by VALU issue (about 85% busy), so this is their time:
+// 1,530 -> 1,288 VALU instructions per wavefront (256^3 MHD shear layer),
+// 2,075 -> 1,893 us per stage for both; hydro (160^3, three directions in one
+// launch) 594 -> 437 us.
+//
+// Chk: pos() takes a value that has to be positive with an exponent in
+// [-256, 255]; num() one that may also be zero (its frexp exponent is 0 then,
+// as it is for NaN and infinities, whose quotients v_div_fixup returns
+// without reading the reciprocal).  With both in range a quotient lies in
+// 2^+-512, far from the exponents v_div_scale acts on (a denormal or inexact
+// residual needs a dividend below 2^-968, an extreme quotient exponents more
+// than 768 apart).
+// The tests are asm volatile so that each is made where its value is computed:
+// written as expressions they were gathered at the end of the block, with
+// every tested value kept in registers until then (162 instead of 126 VGPRs).
+struct Chk {
+  unsigned n = 0, p = 0;
+  __device__ __forceinline__ void num(double x) {
+    unsigned t;
+    asm volatile(
+        "v_frexp_exp_i32_f64 %1, %2\n\tv_add_u32 %1, 0x100, %1\n\tv_or_b32 %0, %0, %1"
+        : "+v"(n), "=&v"(t)
+        : "v"(x));
+  }
+  __device__ __forceinline__ void pos(double x) { high<0xd0100000u>(__double2hiint(x)); }
+  __device__ __forceinline__ void neg(double x) { high<0x50100000u>(__double2hiint(x)); }
+  __device__ __forceinline__ bool bad() const { return (n & ~511u) || (p & 0xe0000000u); }
+
+ private:
+  template <unsigned MINUS>  // -(high word of the smallest value in range)
+  __device__ __forceinline__ void high(int hi) {
+    unsigned t;
+    asm volatile("v_add_u32 %1, %3, %2\n\tv_or_b32 %0, %0, %1"
+                 : "+v"(p), "=&v"(t)
+                 : "v"(hi), "i"(MINUS));
+  }
+};
+
+__device__ __forceinline__ Den64 fden(double b) { return mkden<true>(b); }
+__device__ __forceinline__ double fdiv_(const Den64 &D, double a) {
+  const double m = a * D.r;
+  return __builtin_amdgcn_div_fixup(fma(fma(-D.b, m, a), D.r, m), D.b, a);
+}
+__device__ __forceinline__ double fsqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  g = fma(fma(-g, g, x), h, g);
+  return fma(fma(-g, g, x), h, g);
+}
+// min and max of two numbers, one instruction (the reference's a < b ? a : b
+// takes three; they differ for NaN, which the sweep's cells are tested for,
+// and in the sign of a zero, see cell_faces).  fmin() would add two
+// instructions that quiet signalling NaNs.
+__device__ __forceinline__ double vmin(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double vmax(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double vmax0(double a) {
+  double r;
+  asm("v_max_f64 %0, %1, 0" : "=v"(r) : "v"(a));
+  return r;
+}
+// the sign bit of x, and y with its sign flipped by such a bit: y * sgn(1, x)
+// without the multiplication
+__device__ __forceinline__ unsigned sbit(double x) {
+  return (unsigned)__double2hiint(x) & 0x80000000u;
+}
+__device__ __forceinline__ double flip(double y, unsigned s) {
+  return __hiloint2double((int)((unsigned)__double2hiint(y) ^ s), __double2loint(y));
+}
+// 0.5 + sgn(0.5, x) and 0.5 - sgn(0.5, x) as bit operations on x's high word:
+// 1 or 0 by the sign bit
+__device__ __forceinline__ double wpos(int hi) {
+  return __hiloint2double(~(hi >> 31) & 0x3ff00000, 0);
+}
+__device__ __forceinline__ double wneg(int hi) {
+  return __hiloint2double((hi >> 31) & 0x3ff00000, 0);
+}
+
+// Grid factors of one cell's slopes (k_geo): dxp = xp - x0, bm = x0 - xm,
+// the two limiter ratios, the half widths and, for minmod, the inverse
+// spacings; Dp, Dm, Dab are the denominators with their reciprocals.
+struct Geo {
+  Den64 Dp, Dm, Dab;
+  double cf, cb, hl, hr, ida, idb;
+};
+
+// Limited slope of one variable, modified_mc / minmod with the operations
+// that only move a sign taken out: sig*0.5*(bot+top) = flip(0.5*(bot+top)),
+// sig*cf*bot = cf*|bot|, sig*cb*top = flip(cb*top) (rounding is symmetric).
+template <int LIM>
+__device__ __forceinline__ double fslope(double u0, double u1, double u2, const Geo &G, Chk &k) {
+  if constexpr (LIM == LIM_MINMOD) {
+    const double x = 1.4 * (u2 - u1) * G.idb;
+    const double y = 1.4 * (u1 - u0) * G.ida;
+    const double zn = (u2 - u0) * G.ida * G.idb;
+    k.num(zn);
+    const unsigned s = sbit(x);
+    const double z = fdiv_(G.Dab, zn);
+    return flip(vmax0(vmin(vmin(fabs(x), flip(y, s)), flip(z, s))), s);
+  } else {
+    const double tn = (u1 - u0) * G.Dp.b;
+    k.num(tn);
+    const double top = fdiv_(G.Dm, tn);
+    const double bot = u2 - u1;
+    const unsigned s = sbit(bot);
+    const double m = vmin(vmin(flip(0.5 * (bot + top), s), G.cf * fabs(bot)), flip(G.cb * top, s));
+    // its dividend needs no test: 0 or at least half the smaller of |bot| and
+    // |top|, top in range with tn, bot with the right neighbour's tn
+    return fdiv_(G.Dp, flip(vmax0(m), s));
+  }
+}
+
+// Both face states of a cell, after the e_int guard: FL at its left face, FR
+// at its right one, of d e m1 m2 m3 (b1 b2 b3), with the density's
+// reciprocal for the velocities (DL, DR).  qv, ql, qr as cell_slopes.  The
+// guard's own face values are the Riemann states unless it resets the slopes
+// to zero (then they are the cell's value), so nothing is evaluated twice.
+//
+// A cell with a NaN, an infinity or a -0 is sent to the plain path: vmin and
+// vmax treat those otherwise than the reference's comparisons.  With none of
+// them a slope's zero may have the other sign, which q +- h*S does not show.
+template <bool MAG, int LIM>
+__device__ __forceinline__ void cell_faces(const double qv[9], const double ql[9],
+                                           const double qr[9], const Geo &G, double FL[8],
+                                           double FR[8], Den64 &DL, Den64 &DR, Chk &k) {
+  constexpr int NS = MAG ? 8 : 5;
+  if constexpr (LIM == LIM_FLAT) {
+#pragma unroll
+    for (int s = 0; s < 8; ++s) FL[s] = FR[s] = s < NS ? qv[s] : 0.0;
+    k.pos(qv[0]);
+    DL = DR = fden(qv[0]);
+    return;
+  }
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    if (s >= NS) {
+      FL[s] = FR[s] = 0.0;
+      continue;
+    }
+    const double S = fslope<LIM>(ql[s], qv[s], qr[s], G, k);
+    FL[s] = qv[s] - G.hl * S;
+    FR[s] = qv[s] + G.hr * S;
+    if (s % 4 == 3) fence();
+  }
+  fence();
+  k.pos(FL[0]);
+  k.pos(FR[0]);
+  DL = fden(FL[0]);
+  DR = fden(FR[0]);
+  const double kl = 0.5 * (FL[2] * FL[2] + FL[3] * FL[3] + FL[4] * FL[4]);
+  const double kr = 0.5 * (FR[2] * FR[2] + FR[3] * FR[3] + FR[4] * FR[4]);
+  k.num(kl);
+  k.num(kr);
+  double eintl = FL[1] - fdiv_(DL, kl);
+  double eintr = FR[1] - fdiv_(DR, kr);
+  if (MAG) {
+    eintl = eintl - 0.5 * (FL[5] * FL[5] + FL[6] * FL[6] + FL[7] * FL[7]);
+    eintr = eintr - 0.5 * (FR[5] * FR[5] + FR[6] * FR[6] + FR[7] * FR[7]);
+  }
+  const double el_ = ql[8], em_ = qv[8], er_ = qr[8];
+  if (eintl >= vmax(el_, em_) || eintl <= vmin(el_, em_) || eintr >= vmax(em_, er_) ||
+      eintr <= vmin(em_, er_)) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) FL[s] = FR[s] = qv[s];
+    k.pos(qv[0]);
+    DL = DR = fden(qv[0]);
+  }
+}
+
+// cell values vmin and vmax may not see (NaN, infinity, -0)
+template <bool MAG>
+__device__ __forceinline__ bool odd_cell(const double qv[9]) {
+  bool b = __builtin_amdgcn_class(qv[8], 0x227);
+#pragma unroll
+  for (int s = 0; s < (MAG ? 8 : 5); ++s) b |= __builtin_amdgcn_class(qv[s], 0x227);
+  return b;
+}
+
+// get_cf, the checked fast form; asq = cs*cs is in range (the caller's pos()),
+// so a quotient b*b/d too small for fdiv_ is lost in the sum as it is in the
+// reference's, and one too large shows in the radicand
+__device__ __forceinline__ double fast_cf(const Den64 &Dd, double cs, double b1, double b2,
+                                          double b3, Chk &k) {
+  const double asq = cs * cs;
+  k.pos(asq);
+  const double bb1 = fdiv_(Dd, b1 * b1);
+  const double bb2 = fdiv_(Dd, b2 * b2);
+  const double bb3 = fdiv_(Dd, b3 * b3);
+  const double s = asq + (bb1 + bb2 + bb3);
+  const double r = s * s - 4.0 * asq * bb1;
+  k.pos(r);
+  return fsqrt(0.5 * (s + fsqrt(r)));
+}
+
+// hlldflux + fstar as hlld(), in the checked fast form.  Dch: ch with its
+// reciprocal.  Hydro (MAG false): with B = 0 and psi = 0 the transverse
+// states, the Alfven states and every term with b1 are the identity or a
+// zero, and both Alfven speeds are sm, so only the contact's selection is
+// left; what changes is the sign of a zero flux, which no update of a state
+// without -0 shows.
+template <bool MAG>
+__device__ __forceinline__ void hlld_fast(double f[9], double cfl, double cfr, double v1l,
+                                          double v1r, double v2l, double v2r, double v3l,
+                                          double v3r, double dl, double dr, double el, double er,
+                                          double ptl, double ptr, double b1l, double b1r,
+                                          double b2l, double b2r, double b3l, double b3r,
+                                          double phil, double phir, const Den64 &Dch, Chk &k) {
+  const double sl = vmin(vmin(v1r - cfr, v1l - cfl), 0.0);
+  const double sr = vmax(vmax(v1r + cfr, v1l + cfl), 0.0);
+  const double slv = sl - v1l, srv = sr - v1r;
+  const double den = srv * dr - slv * dl;
+  k.pos(den);
+  const Den64 Dden = fden(den);
+  const double smn = srv * dr * v1r - slv * dl * v1l - ptr + ptl;
+  const double pan = srv * dr * ptl - slv * dl * ptr + dl * dr * srv * slv * (v1r - v1l);
+  k.num(smn);
+  k.num(pan);
+  const double sm = fdiv_(Dden, smn), pta = fdiv_(Dden, pan);
+  const double slm = sl - sm, srm = sr - sm;
+  k.neg(slm);
+  k.pos(srm);
+  const Den64 Dslm = fden(slm), Dsrm = fden(srm);
+  const double dla = fdiv_(Dslm, dl * slv), dra = fdiv_(Dsrm, dr * srv);
+  k.pos(dla);
+  k.pos(dra);
+  fence();
+  const int hsm = __double2hiint(sm);
+  if constexpr (!MAG) {
+    const double eln = slv * el - ptl * v1l + pta * sm, ern = srv * er - ptr * v1r + pta * sm;
+    k.num(eln);
+    k.num(ern);
+    const double ela = fdiv_(Dslm, eln), era = fdiv_(Dsrm, ern);
+    const double wl = wpos(hsm), wr = wneg(hsm);
+    const double d_ = wl * dla + wr * dra;
+    f[0] = d_ * sm;
+    f[1] = d_ * sm * sm + pta;
+    f[2] = d_ * sm * (wl * v2l + wr * v2r);
+    f[3] = d_ * sm * (wl * v3l + wr * v3r);
+    f[4] = ((wl * ela + wr * era) + pta) * sm;
+    f[5] = f[6] = f[7] = f[8] = 0.0;
+    return;
+  }
+  const double ch = Dch.b;
+  const double dphi = phir - phil;
+  k.num(dphi);
+  k.pos(ch);
+  const double b1 = 0.5 * ((b1l + b1r) - fdiv_(Dch, dphi));
+  const double phi = 0.5 * ((phil + phir) - (b1r - b1l) * ch);
+
+  const double sqla = fsqrt(dla), sqra = fsqrt(dra);
+  const double ab1 = fabs(b1);
+  k.num(b1);
+  const double sla = sm - fdiv_(fden(sqla), ab1);
+  const double sra = sm + fdiv_(fden(sqra), ab1);
+
+  const double b1b1 = b1 * b1;
+  const double dnl = dl * slv * slm - b1b1, dnr = dr * srv * srm - b1b1;
+  k.pos(dnl);
+  k.pos(dnr);
+  const Den64 Dl = fden(dnl), Dr = fden(dnr);
+  auto qd = [&](const Den64 &D, double a) {
+    k.num(a);
+    return fdiv_(D, a);
+  };
+  const double v2la = v2l - qd(Dl, b1 * b2l * (sm - v1l));
+  const double v2ra = v2r - qd(Dr, b1 * b2r * (sm - v1r));
+  const double v3la = v3l - qd(Dl, b1 * b3l * (sm - v1l));
+  const double v3ra = v3r - qd(Dr, b1 * b3r * (sm - v1r));
+  const double numl = dl * slv * slv - b1b1;
+  const double numr = dr * srv * srv - b1b1;
+  const double b2la = qd(Dl, b2l * numl);
+  const double b2ra = qd(Dr, b2r * numr);
+  const double b3la = qd(Dl, b3l * numl);
+  const double b3ra = qd(Dr, b3r * numr);
+  fence();
+
+  const double ela = qd(Dslm, slv * el - ptl * v1l + pta * sm +
+                                  b1 * ((v1l * b1 + v2l * b2l + v3l * b3l) -
+                                        (sm * b1 + v2la * b2la + v3la * b3la)));
+  const double era = qd(Dsrm, srv * er - ptr * v1r + pta * sm +
+                                  b1 * ((v1r * b1 + v2r * b2r + v3r * b3r) -
+                                        (sm * b1 + v2ra * b2ra + v3ra * b3ra)));
+
+  fence();
+  const unsigned s1 = sbit(b1);
+  const Den64 Dsqs = fden(sqla + sqra);
+  const double v2aa = qd(Dsqs, sqla * v2la + sqra * v2ra + flip(b2ra - b2la, s1));
+  const double v3aa = qd(Dsqs, sqla * v3la + sqra * v3ra + flip(b3ra - b3la, s1));
+  const double sqp = fsqrt(dla * dra);
+  const double b2aa = qd(Dsqs, sqla * b2ra + sqra * b2la + flip(sqp * (v2ra - v2la), s1));
+  const double b3aa = qd(Dsqs, sqla * b3ra + sqra * b3la + flip(sqp * (v3ra - v3la), s1));
+
+  fence();
+  const double vbaa = v2aa * b2aa + v3aa * b3aa;
+  const double eraa = era + flip(sqra * ((v2ra * b2ra + v3ra * b3ra) - vbaa), s1);
+  const double elaa = ela - flip(sqla * ((v2la * b2la + v3la * b3la) - vbaa), s1);
+
+  const int hla = __double2hiint(sla), hra = __double2hiint(sra);
+  const double wl = wpos(hla), wr = wneg(hra), wa = wneg(hla ^ hra);
+  const double d_ = wpos(hsm) * dla + wneg(hsm) * dra;
+  const double v2_ = wl * v2la + wa * v2aa + wr * v2ra;
+  const double v3_ = wl * v3la + wa * v3aa + wr * v3ra;
+  const double b2_ = wl * b2la + wa * b2aa + wr * b2ra;
+  const double b3_ = wl * b3la + wa * b3aa + wr * b3ra;
+  const double e_ = wl * ela + wneg(hla ^ hsm) * elaa + wneg(hsm ^ hra) * eraa + wr * era;
+  f[0] = d_ * sm;
+  f[1] = d_ * sm * sm + pta - b1b1;
+  f[2] = d_ * sm * v2_ - b1 * b2_;
+  f[3] = d_ * sm * v3_ - b1 * b3_;
+  f[4] = (e_ + pta) * sm - b1 * (sm * b1 + v2_ * b2_ + v3_ * b3_);
+  f[5] = phi;
+  f[6] = b2_ * sm - b1 * v2_;
+  f[7] = b3_ * sm - b1 * v3_;
+  f[8] = ch * ch * b1;
+}
+
+// Face states to flux, as face_flux: L the left cell's FR, R_ the right
+// cell's FL, Dl and Dr their densities' reciprocals; fe: dl eil dr eir.
+template <int DIR, bool MAG>
+__device__ __forceinline__ void face_fast(const double L[8], const double R_[8], double phil,
+                                          double phir, const Den64 &Dl, const Den64 &Dr,
+                                          double gam, const Den64 &Dch, double t[9], double fe[4],
+                                          Chk &k) {
+  constexpr int a_ = DIR, b_ = (DIR + 1) % 3, c_ = (DIR + 2) % 3;
+  auto qd = [&](const Den64 &D, double a) {
+    k.num(a);
+    return fdiv_(D, a);
+  };
+  const double v1l = qd(Dl, L[2 + a_]), v1r = qd(Dr, R_[2 + a_]);
+  const double v2l = qd(Dl, L[2 + b_]), v2r = qd(Dr, R_[2 + b_]);
+  const double v3l = qd(Dl, L[2 + c_]), v3r = qd(Dr, R_[2 + c_]);
+  double b1l = 0, b1r = 0, b2l = 0, b2r = 0, b3l = 0, b3r = 0;
+  if (MAG) {
+    b1l = L[5 + a_];
+    b1r = R_[5 + a_];
+    b2l = L[5 + b_];
+    b2r = R_[5 + b_];
+    b3l = L[5 + c_];
+    b3r = R_[5 + c_];
+  }
+  const double eil = get_eint(MAG, L[1], L[0], v1l, v2l, v3l, b1l, b2l, b3l);
+  const double eir = get_eint(MAG, R_[1], R_[0], v1r, v2r, v3r, b1r, b2r, b3r);
+  fe[0] = L[0];
+  fe[1] = eil;
+  fe[2] = R_[0];
+  fe[3] = eir;
+  fence();
+  double ptl = (gam - 1.0) * eil, ptr = (gam - 1.0) * eir;
+  // quotients in range (pos) with the density in range: so was the dividend
+  const double asl = fdiv_(Dl, gam * ptl), asr = fdiv_(Dr, gam * ptr);
+  k.pos(asl);
+  k.pos(asr);
+  double cfl = fsqrt(asl), cfr = fsqrt(asr);
+  if (MAG) {
+    ptl = ptl + 0.5 * (b1l * b1l + b2l * b2l + b3l * b3l);
+    ptr = ptr + 0.5 * (b1r * b1r + b2r * b2r + b3r * b3r);
+    cfl = fast_cf(Dl, cfl, b1l, b2l, b3l, k);
+    cfr = fast_cf(Dr, cfr, b1r, b2r, b3r, k);
+  }
+  fence();
+  // without B get_cf is sqrt(0.5*(cs^2 + sqrt(cs^4))) = cs exactly: the
+  // square root of a rounded square is the number itself
+  hlld_fast<MAG>(t, cfl, cfr, v1l, v1r, v2l, v2r, v3l, v3r, L[0], R_[0], L[1], R_[1], ptl, ptr,
+                 b1l, b1r, b2l, b2r, b3l, b3r, phil, phir, Dch, k);
 }
 
 // ---- FP32-mixed HLLD in perturbation form ----------------------------------
