@@ -45,7 +45,9 @@ struct hg_ctx {
   std::vector<int> ev_kind;     // kind of each recorded pair
   int ev_used = 0;
   KEv kev{};
-  bool fused = false;   // last sweep direction fused with the RK update
+  // one sweep direction (D.fdir) fused with the RK update; auto_form: as
+  // default_form chose, until hg_set_fused says otherwise
+  bool fused = false, auto_form = true;
   long part_cap = 0;    // CFL partial slots allocated
   // the second state buffer set of the fused form (W aliasing U as in D)
   double *alt_U[NVMAX] = {}, *alt_W[NWMAX] = {};
@@ -128,6 +130,45 @@ static int validate(const hg_desc *d) {
   for (auto a : arr)
     if (!*a) return HG_ERR_ARG;
   return HG_OK;
+}
+
+// A batch member's own steps (outside the batch) take the separate form: the
+// batch numbers its state sets.
+static bool fused_now(const hg_ctx *c) { return c->fused && !c->in_batch; }
+
+static int fused_direction(const hg_ctx *c, int32_t on);
+static int ensure_fused_buffers(hg_ctx *c, int L);
+
+// The form a context starts with (hg_set_fused changes it; the results are the
+// same bits).  1D boxes: their one direction is fused, a stage is then one
+// launch instead of two (Sod 500: 30.6 -> 24.6 us per step, 1D MHD 1001: 50 ->
+// 34).  2D and 3D boxes with x: x is fused from 2^15 (2D) and 2^17 cells (3D)
+// on.  There the divergence that stays out of memory and the smaller kernels
+// count (512^2 176 -> 136 us per step, 192^2 69 -> 63, 64^3 242 -> 207,
+// 97x131x75 978 -> 632, 160^3 hydro 1333 -> 979); below, the one launch for
+// all directions does (160^2 59 against 61, 48^3 even, 40^3 90 against 114).
+// Without x (a y-z plane) the separate form is faster (512^2: 264 against 530).
+// A box whose further state sets do not fit keeps the separate form.
+static void default_form(hg_ctx *c) {
+  const Dev &D = c->D;
+  const int on = D.dim == 1 ? (D.solve[0] ? 2 : 1) : 2;
+  if (D.dim == 0 || (D.dim == 2 && D.ncell < 1 << 15) || (D.dim == 3 && D.ncell < 1 << 17)) return;
+  const int L = fused_direction(c, on);
+  if (L < 0) return;
+  const size_t held = c->allocs.size();
+  double *const part = D.part;
+  const long cap = c->part_cap;
+  if (ensure_fused_buffers(c, L) != HG_OK) {
+    (void)hipGetLastError();
+    for (size_t q = held; q < c->allocs.size(); ++q) hipFree(c->allocs[q]);
+    c->allocs.resize(held);
+    c->alt_ready = c->alt2_ready = false;
+    c->D.part = part;
+    c->part_cap = cap;
+    return;
+  }
+  c->D.fdir = L;
+  c->fused = true;
 }
 
 extern "C" int hg_create(const hg_desc *desc, hg_ctx **out) {
@@ -380,6 +421,7 @@ extern "C" int hg_create(const hg_desc *desc, hg_ctx **out) {
     return fail(HG_ERR_NOMEM);
   if (hipHostMalloc((void **)&c->h_stage, fb, hipHostMallocDefault) != hipSuccess)
     return fail(HG_ERR_NOMEM);
+  default_form(c);
   *out = c;
   return HG_OK;
 }
@@ -619,7 +661,8 @@ extern "C" int hg_profile_read(const hg_ctx *c, int32_t kind, double *ms_total,
   const int wr = D.nw - (D.mag ? 5 : 2);
   // directions the sweep launches cover: every solved one, or all but the
   // fused one
-  const int nsw = D.dim - (c->fused ? 1 : 0);
+  const bool fused = fused_now(c);
+  const int nsw = D.dim - (fused ? 1 : 0);
   double bytes = 0.0;
   switch (kind) {
     case HG_PROF_SWEEP:  // read the primitives once and write one divergence per direction
@@ -632,7 +675,7 @@ extern "C" int hg_profile_read(const hg_ctx *c, int32_t kind, double *ms_total,
       // divergence, and with its three state sets stage 1 neither reads
       // nor writes a U0 (averaged over the stages)
       const int rk = c->desc.rktype;
-      bytes = cell * (c->fused ? D.nw + nsw * D.nv + 2.0 * D.nv +
+      bytes = cell * (fused ? D.nw + nsw * D.nv + 2.0 * D.nv +
                                      (double)D.nv * (rk - 1) / rk + wr
                                : (double)(D.dim * D.nv + 3 * D.nv + wr));
       break;
@@ -780,13 +823,23 @@ extern "C" int hg_gravity(hg_ctx *c, double time, double dt, double *grvtime, do
   return HG_OK;
 }
 
+// The roles of the fused form's state sets after one step: the set the last
+// stage wrote (the second for one or three stages, the third for two) trades
+// places with the current one.  Turning twice changes nothing.
+static void turn_sets(hg_ctx *c) {
+  double **U = c->desc.rktype % 2 == 1 ? c->alt_U : c->D.U0;
+  double **W = c->desc.rktype % 2 == 1 ? c->alt_W : c->alt2_W;
+  for (int v = 0; v < c->D.nv; ++v) std::swap(c->D.U[v], U[v]);
+  for (int w = 0; w < c->D.nw; ++w) std::swap(c->D.W[w], W[w]);
+}
+
 // The part of RK stage 1 that needs neither the step's dt nor the gravity
 // potential of this step: the flux sweep (of every direction, or of the
 // directions before the fused one) and the species pass.  It only reads the
 // primitives and ch, which the previous step's end has already set.
 static void enqueue_stage1_sweep(hg_ctx *c) {
   const Dev &D = c->D;
-  if (c->fused) {
+  if (fused_now(c)) {
     RKArgs a{};
     launch_fused_stage(D, 1, a, c->stream, nullptr, nullptr, 1);
     return;
@@ -803,9 +856,10 @@ static int enqueue_stages(hg_ctx *c, bool fuse_tail, double damp, bool sweep1_do
   const Dev &D = c->D;
   const int rk = c->desc.rktype;
   int npart = D.nblk_cfl;
+  const bool fused = fused_now(c);
   // the fused form's three state sets (current, second, third)
   StateSet cur{}, alt{}, third{};
-  if (c->fused) {
+  if (fused) {
     for (int v = 0; v < D.nv; ++v) {
       cur.U[v] = c->D.U[v];
       alt.U[v] = c->alt_U[v];
@@ -821,7 +875,7 @@ static int enqueue_stages(hg_ctx *c, bool fuse_tail, double damp, bool sweep1_do
     double faco, fact, facn;
     runge_coeff(stage, rk, &faco, &fact, &facn);
     const bool pre = sweep1_done && stage == 1;
-    if (c->fused) {
+    if (fused) {
       const bool last = stage == rk;
       RKArgs a{faco, fact, facn, damp, fuse_tail && last, fuse_tail && last && damp > 0.0,
                D.grav};
@@ -860,24 +914,9 @@ static int enqueue_stages(hg_ctx *c, bool fuse_tail, double damp, bool sweep1_do
     launch_rk(D, stage, faco, fact, facn, fuse_tail && last, fuse_tail && last && damp > 0.0,
               damp, c->stream, prof_ev(c, HG_PROF_RK));
   }
-  if (c->fused) {
-    // the last stage's output becomes the current set; the step's starting
-    // set is free again and takes the role its slot had
-    const bool in_alt = rk % 2 == 1;
-    const StateSet &ncur = in_alt ? alt : third;
-    const StateSet &nalt = in_alt ? cur : alt;
-    const StateSet &nthird = in_alt ? third : cur;
-    for (int v = 0; v < D.nv; ++v) {
-      c->D.U[v] = ncur.U[v];
-      c->alt_U[v] = nalt.U[v];
-      c->D.U0[v] = nthird.U[v];
-    }
-    for (int w = 0; w < D.nw; ++w) {
-      c->D.W[w] = ncur.W[w];
-      c->alt_W[w] = nalt.W[w];
-      c->alt2_W[w] = nthird.W[w];
-    }
-  }
+  // the last stage's output becomes the current set; the step's starting
+  // set is free again and takes the role its slot had
+  if (fused) turn_sets(c);
   return npart;
 }
 
@@ -947,6 +986,10 @@ extern "C" int hg_run(hg_ctx *c, double *time, int64_t *tn, double *t_out, doubl
     // number of event pairs)
     const int64_t ran = c->h_sc->tn - tn_before;
     tn_before = c->h_sc->tn;
+    // steps enqueued after the stop left the state sets alone (a step that
+    // ends in an error has run)
+    const int64_t idle = nb - ran - (c->h_sc->stop == STOP_ERROR ? 1 : 0);
+    if (fused_now(c) && idle % 2 != 0) turn_sets(c);
     if (c->prof)
       c->ev_used = ev_base + (int)(std::min<int64_t>(ran, nb) * ((c->ev_used - ev_base) / nb));
     prof_collect(c);
@@ -1203,35 +1246,40 @@ static void member_to_set(hg_ctx *c, int p) {
   put_sets(c, c->bsets[p], c->bsets[(p + 1) % 3], c->bsets[(p + 2) % 3]);
 }
 
+// The direction hg_set_fused's `on` (1 the last solved direction, y or z; 2
+// x) fuses, or -1 where the context does not take that form: the fused
+// kernels carry no species and the boundary codes 0-3 only.
+static int fused_direction(const hg_ctx *c, int32_t on) {
+  const Dev &D = c->D;
+  int L = -1;
+  if (on == 2) L = D.solve[0] ? 0 : -1;
+  else
+    for (int a = 1; a < 3; ++a)
+      if (D.solve[a]) L = a;
+  if (D.nspc) return -1;
+  for (int a = 0; a < 3; ++a)
+    if (D.ax[a].ext) return -1;
+  return L;
+}
+
 extern "C" int hg_set_fused(hg_ctx *c, int32_t on) {
   if (!c) return HG_ERR_ARG;
   HIPCHK(hipSetDevice(c->device));
   HIPCHK(hipStreamSynchronize(c->stream));
   Dev &D = c->D;
   if (!on) {
-    c->fused = false;
+    c->fused = c->auto_form = false;
     D.fdir = -1;
     return HG_OK;
   }
-  // no species; on = 1: the last solved direction (y or z),
-  // on = 2: x
-  int L = -1;
-  if (on == 2) {
-    L = D.solve[0] ? 0 : -1;
-  } else if (on == 1) {
-    for (int a = 1; a < 3; ++a)
-      if (D.solve[a]) L = a;
-  } else {
-    return HG_ERR_ARG;
-  }
-  if (D.nspc || L < 0) return HG_ERR_UNSUPPORTED;
-  for (int a = 0; a < 3; ++a)
-    if (D.ax[a].ext) return HG_ERR_UNSUPPORTED;  // fused kernels carry codes 0-3 only
-  if (c->in_batch) return HG_ERR_UNSUPPORTED;
+  if (on != 1 && on != 2) return HG_ERR_ARG;
+  const int L = fused_direction(c, on);
+  if (L < 0 || c->in_batch) return HG_ERR_UNSUPPORTED;
   int st = ensure_fused_buffers(c, L);
   if (st) return st;
   D.fdir = L;
   c->fused = true;
+  c->auto_form = false;
   return HG_OK;
 }
 
@@ -1409,7 +1457,7 @@ extern "C" int hg_batch_add(hg_batch *b, hg_ctx *c, double time, double t_out, d
                             int64_t tn_out) {
   if (!b || !c) return HG_ERR_ARG;
   if (c->device != b->device || c->D.grav || c->D.nspc || c->D.ax[0].ext || c->D.ax[1].ext ||
-      c->D.ax[2].ext || c->fused)
+      c->D.ax[2].ext || (c->fused && !c->auto_form))
     return HG_ERR_UNSUPPORTED;
   for (hg_ctx *m : b->members)
     if (m == c) return HG_ERR_ARG;

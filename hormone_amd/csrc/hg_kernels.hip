@@ -1466,19 +1466,7 @@ __device__ __forceinline__ void fused_rk(const Dev &D, const Axis &A, long base,
 template <int DIR, bool MAG, int LIM, bool TILE, bool MIX = false>
 __global__ __launch_bounds__(1024) void k_sweep_rk(Dev D, int stage, RKArgs rk) {
   extern __shared__ double lds[];
-  if (gptr(D.sc)->stop) {
-    // stages enqueued after the run stopped: the host still makes the
-    // output set the current one, so hand the state over unchanged
-    const long nt = (long)gridDim.x * blockDim.x;
-    for (long m = (long)blockIdx.x * blockDim.x + threadIdx.x; m < D.ncell; m += nt) {
-      for (int v = 0; v < D.nv; ++v) gptr(D.Uo[v])[m] = gptr(D.U[v])[m];
-      for (int w = 0; w < D.nw; ++w) {  // d, e, B alias U; a shared phi stays
-        const bool aliased = w == WD || w == WE || (MAG && w >= WB1 && w <= WB3);
-        if (!aliased && D.Wo[w] != D.W[w]) gptr(D.Wo[w])[m] = gptr(D.W[w])[m];
-      }
-    }
-    return;
-  }
+  if (gptr(D.sc)->stop) return;
   const int lane = threadIdx.x & 63;
   const long wave = (long)blockIdx.x * (blockDim.x >> 6) + wave_in_block();
   double dti = __builtin_inf(), cfm = 0.0;

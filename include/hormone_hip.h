@@ -263,15 +263,19 @@ int hg_set_ghosts(hg_ctx *ctx, int32_t field, const double *padded);
 int hg_set_boundary_flux(hg_ctx *ctx, int32_t face, const double *flux);
 
 /* Fuse one direction's sweep with the RK update: on = 1 the last solved
-   direction (y or z), on = 2 the x direction, 0 off (the default).  One
+   direction (y or z), on = 2 the x direction, 0 off.  A new context takes
+   the form that is faster for its shape and size (1D boxes their one
+   direction, 2D boxes from 2^15 and 3D boxes from 2^17 cells on x), and
+   keeps it until this call.  One
    launch per RK stage does that direction's reconstruction, Riemann solves
    and flux difference and updates each cell, so that direction's flux
    divergence is never written to or read back from HBM; the other
    directions are swept first.  Results are bit-identical either way, in
    FP64 and FP32-mixed.  Not with species, boundary codes 4, 5, 9, 10 or
-   while the context is in a batch (HG_ERR_UNSUPPORTED).  The first call allocates a second copy
-   of the state (the launch reads one and writes the other).  No
-   counterpart in the reference (a launch-shape choice). */
+   while the context is in a batch (HG_ERR_UNSUPPORTED).  A context that
+   starts separate allocates the further copies of the state at the first
+   call (the launch reads one and writes another).  No counterpart in the
+   reference (a launch-shape choice). */
 int hg_set_fused(hg_ctx *ctx, int32_t on);
 
 /* The sweep kernel's duration without per-dispatch events: `launches`
