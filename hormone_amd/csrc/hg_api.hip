@@ -195,6 +195,7 @@ extern "C" int hg_create(const hg_desc *desc, hg_ctx **out) {
   D.n1 = desc->ie - desc->is + 1;
   D.n2 = desc->je - desc->js + 1;
   D.n3 = desc->ke - desc->ks + 1;
+  D.n1_inv = (unsigned)std::min<unsigned long long>((1ull << 32) / (unsigned)D.n1, 0xffffffffull);
   c->nxg = D.n1 + 4;
   c->nyg = D.n2 + 4;
   c->nzg = D.n3 + 4;
@@ -243,6 +244,7 @@ extern "C" int hg_create(const hg_desc *desc, hg_ctx **out) {
       A.idx = dp[4];
       A.idxi = dp[5];
       A.n = nn[a];
+      A.n4_inv = (unsigned)((1ull << 32) / (unsigned)(nn[a] + 4));
       A.nlines = (unsigned)(D.ncell / nn[a]);
       // x lines form one sweep sequence, y and z lines one per column i
       A.nsub = a == 0 ? A.nlines : A.nlines / (unsigned)D.n1;
@@ -258,7 +260,7 @@ extern "C" int hg_create(const hg_desc *desc, hg_ctx **out) {
         hipStreamSynchronize(c->stream) != hipSuccess)
       return fail(HG_ERR_DEVICE);
     // the FP64 slopes' grid factors; the fast divisions rely on spacings
-    // within 2^+-100 and limiter ratios within 2^+-8 (cell_faces, fslope)
+    // within 2^+-100 and limiter ratios within 2^+-8 (Chk, fslope)
     for (int a = 0; a < 3; ++a) {
       const int m = nn[a] + 4;
       double2 *geo = nullptr;

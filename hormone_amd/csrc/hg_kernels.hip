@@ -49,6 +49,14 @@ __device__ __forceinline__ int wave_in_block() {
   return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 }
 
+// The lane's index, computed where it is asked for: a value kept from the start
+// of a sweep takes a register the solver needs.
+__device__ __forceinline__ int lane_again() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t & 63;
+}
+
 struct Cell {
   double d, v[3], e, eint, b[3], phi;
 };
@@ -301,7 +309,9 @@ __device__ __forceinline__ void park_cell(double *lds, const Cell &q) {
 }
 template <bool MAG>
 __device__ __forceinline__ Cell parked_cell(const double *lds) {
-  const double *p = lds + threadIdx.x;
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));  // the addresses again, not kept from park_cell
+  const double *p = lds + t;
   const int bs = blockDim.x;
   Cell q;
   q.d = p[0];
@@ -333,17 +343,9 @@ __device__ __forceinline__ Cell parked_cell(const double *lds) {
 // c (-2 .. n+1) of the position; false past the sequence's end, where c is
 // n+1 of the last line and the lane stores nothing.
 template <int DIR>
-__device__ __forceinline__ bool lane_cell(const Dev &D, const Axis &A, long w, int r,
-                                          long &line, long &base, int &c) {
-  const unsigned n4 = (unsigned)A.n + 4u;
-  unsigned col = 0, s = (unsigned)w;
-  if (DIR != 0) {
-    col = (unsigned)w % (unsigned)D.n1;
-    s = (unsigned)w / (unsigned)D.n1;
-  }
-  const unsigned pos = s * (unsigned)SEG + (unsigned)r;
-  unsigned sub = pos / n4;
-  c = (int)(pos - sub * n4) - 2;
+__device__ __forceinline__ bool place_cell(const Dev &D, const Axis &A, unsigned col, unsigned sub,
+                                           unsigned off, long &line, long &base, int &c) {
+  c = (int)off - 2;
   const bool in = sub < A.nsub;
   if (!in) {
     sub = A.nsub - 1;
@@ -357,6 +359,55 @@ __device__ __forceinline__ bool lane_cell(const Dev &D, const Axis &A, long w, i
     base = DIR == 1 ? (long)col + (long)sub * D.n1 * D.n2 : line;
   }
   return in;
+}
+
+// u / d with inv = the host's floor(2^32 / d), and the remainder: mulhi is the
+// quotient or one less
+__device__ __forceinline__ unsigned udiv(unsigned u, unsigned d, unsigned inv, unsigned &rem) {
+  unsigned q = __umulhi(u, inv);
+  rem = u - q * d;
+  if (rem >= d) {
+    ++q;
+    rem -= d;
+  }
+  return q;
+}
+
+// w is the same for the whole wavefront: both divisions run on the scalar unit
+// for lane 0, and the other lanes' positions follow by one subtraction (lines
+// shorter than a wavefront divide their own).
+template <int DIR>
+__device__ __forceinline__ bool lane_cell(const Dev &D, const Axis &A, long w, int r,
+                                          long &line, long &base, int &c) {
+  const unsigned n4 = (unsigned)A.n + 4u;
+  const unsigned uw = (unsigned)__builtin_amdgcn_readfirstlane((int)w);
+  unsigned col = 0, s = uw;
+  if (DIR != 0) s = udiv(uw, (unsigned)D.n1, D.n1_inv, col);
+  unsigned off;
+  unsigned sub = udiv(s * (unsigned)SEG, n4, A.n4_inv, off);
+  off += (unsigned)r;
+  if (n4 >= 64u) {
+    const bool next = off >= n4;
+    sub += next ? 1u : 0u;
+    off -= next ? n4 : 0u;
+  } else {
+    unsigned rem;
+    sub += udiv(off, n4, A.n4_inv, rem);
+    off = rem;
+  }
+  return place_cell<DIR>(D, A, col, sub, off, line, base, c);
+}
+
+// the same for a wave of the thread's own
+template <int DIR>
+__device__ __forceinline__ bool thread_cell(const Dev &D, const Axis &A, long w, int r,
+                                            long &line, long &base, int &c) {
+  const unsigned n4 = (unsigned)A.n + 4u;
+  const unsigned col = DIR != 0 ? (unsigned)w % (unsigned)D.n1 : 0u;
+  const unsigned s = DIR != 0 ? (unsigned)w / (unsigned)D.n1 : (unsigned)w;
+  const unsigned pos = s * (unsigned)SEG + (unsigned)r;
+  const unsigned sub = pos / n4;
+  return place_cell<DIR>(D, A, col, sub, pos - sub * n4, line, base, c);
 }
 
 // cell-0 coordinates of a line (error reports)
@@ -382,11 +433,11 @@ __device__ __forceinline__ void cell_ijk(const Dev &D, long m, int &i, int &j, i
   k = (int)kk;
 }
 
-// the lane's own cell of a loaded tile (zero: 0, see sweep_line)
+// the lane's own cell of a loaded tile
 template <int DIR, bool MAG>
 __device__ __forceinline__ Cell tile_column(const Dev &D, const Axis &A, int c,
-                                            const double *lds, int zero = 0) {
-  const int bw = blockDim.x >> 6, w = threadIdx.x >> 6, lane = (threadIdx.x & 63) + zero;
+                                            const double *lds) {
+  const int bw = blockDim.x >> 6, w = wave_in_block(), lane = lane_again();
   const int ld = tile_ld(bw), fs = 64 * ld;
   const int nf = MAG ? NWMAX : WEINT + 1;
   double f[NWMAX];
@@ -424,7 +475,7 @@ __device__ __forceinline__ Cell tile_cell(const Dev &D, const Axis &A, long wave
       const long wc = wave0 + col < last ? wave0 + col : last;
       long ln, bc;
       int cl;
-      lane_cell<DIR>(D, A, wc, r, ln, bc, cl);
+      thread_cell<DIR>(D, A, wc, r, ln, bc, cl);
       double f[NWMAX];
       raw_cell<DIR, MAG>(D, A, bc, ln, cl, f);
 #pragma unroll
@@ -474,17 +525,21 @@ __device__ __forceinline__ void store_du(const Dev &D, const Axis &A, long base,
     }
     return;
   }
-  const int bw = blockDim.x >> 6, w = threadIdx.x >> 6;
+  // the tile addresses computed again: kept from the load they took registers
+  // the solver needs (9 spills)
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  const int bw = blockDim.x >> 6, w = t >> 6;
   const int ld = tile_ld(bw), fs = 64 * ld;
   __syncthreads();  // every wavefront has read its cells out of the tile
   {
-    double *p = lds + lane * ld + w;
+    double *p = lds + (t & 63) * ld + w;
 #pragma unroll
     for (int v = 0; v < NVMAX; ++v)
       if (v < nv) p[v * fs] = du[v];
   }
   __syncthreads();
-  const int t = threadIdx.x, r = t >> __builtin_ctz(bw), col = t & (bw - 1);
+  const int r = t >> __builtin_ctz(bw), col = t & (bw - 1);
   long m;
   if (tile_row_cell<MAG>(lds, bw, t, m)) {
     const double *p = lds + r * ld + col;
@@ -708,9 +763,8 @@ __device__ __forceinline__ Geo load_geo(const Axis &A, int c) {
 // (checked fast form).  True, for the whole wavefront, when one of its
 // faces -1 .. n-1 depends on a value out of the fast form's range.
 template <int DIR, bool MAG, int LIM>
-__device__ __forceinline__ bool line_faces(const Axis &A, const Cell &q, int c, int cc, int lane,
-                                           double gam, const Den64 &Dch, double t[9],
-                                           double fe[4]) {
+__device__ __forceinline__ bool line_faces(const Axis &A, const Cell &q, int c, int lane,
+                                           double gam, const Den64 &Dch, double t[9]) {
   const int n = A.n;
   double qv[9], ql[9], qr[9];
   slope_values<MAG>(q, qv);
@@ -722,14 +776,13 @@ __device__ __forceinline__ bool line_faces(const Axis &A, const Cell &q, int c, 
       qr[s] = dn1(qv[s]);
     }
   }
-  const Geo G = load_geo<LIM>(A, cc);
+  const Geo G = load_geo<LIM>(A, c);
   double FL[8], FR[8], R_[8];
   Den64 DL, DR, Dr;
   Chk kc;
   cell_faces<MAG, LIM>(qv, ql, qr, G, FL, FR, DL, DR, kc);
-  // lane 0 has no left neighbour; a slope of cell n also relies on the tests
-  // of cell n+1 (fslope)
-  bad |= __builtin_amdgcn_ballot_w64(c >= -1 && lane >= 1 && kc.bad());
+  // the cells whose faces are used (lane 0 has no left neighbour)
+  bad |= __builtin_amdgcn_ballot_w64(c >= -1 && c <= n && lane >= 1 && lane <= 62 && kc.bad());
   // the right cell's left face state from lane+1
 #pragma unroll
   for (int s = 0; s < 8; ++s) R_[s] = (!MAG && s >= 5) ? 0.0 : dn1(FL[s]);
@@ -738,9 +791,13 @@ __device__ __forceinline__ bool line_faces(const Axis &A, const Cell &q, int c, 
   const double phil = MAG ? q.phi + 0.0 : 0.0;
   const double phir = MAG ? dn1(phil) : 0.0;
   Chk kf;
-  face_fast<DIR, MAG>(FR, R_, phil, phir, DR, Dr, gam, Dch, t, fe, kf);
+  face_fast<DIR, MAG>(FR, R_, phil, phir, DR, Dr, gam, Dch, t, kf);
+  // the fluxes now: they would be put off past the branch to the plain form,
+  // with all they come from kept until there
+#pragma unroll
+  for (int s = 0; s < (MAG ? 9 : 5); ++s) asm volatile("" : "+v"(t[s]));
   bad |= __builtin_amdgcn_ballot_w64(c >= -1 && c <= n - 1 && lane >= 1 && lane <= 61 && kf.bad());
-  return bad != 0 || !A.fast;
+  return bad != 0 || !A.fast || !(Dch.b > 0x1p-256 && Dch.b < 0x1p255);
 }
 
 // The same in plain divisions and square roots.
@@ -810,28 +867,39 @@ __device__ __forceinline__ void sweep_line(const Dev &D, long wave, int lane, in
   const Cell q = TILE ? tile_cell<DIR, MAG, EXT>(D, A, wave0, base, c, valid, lds)
                       : load_cell<DIR, MAG, EXT>(D, A, base, line, c);
   if (FUSED && !TILE) park_cell<MAG>(lds, q);
-  const int cc = c < -2 ? -2 : (c > n + 1 ? n + 1 : c);
+  // (element indices fit in 32 bits)
+  const unsigned ubase = (unsigned)base;
   const double gam = D.gamma;
   const Den64 Dch{gptr(D.sc)->ch, gptr(D.sc)->chr};
-  double t[9], fe[4];
-  const bool odd = line_faces<DIR, MAG, LIM>(A, q, c, cc, lane, gam, Dch, t, fe);
+  double t[9];
+  bool neg = false;  // a face density or internal energy is not positive
+  const bool odd = line_faces<DIR, MAG, LIM>(A, q, c, lane, gam, Dch, t);
+  // the rare branches place the lane again, so that nothing is kept for them
+  auto again = [&](long &line2, long &base2, int &c2) {
+    lane_cell<DIR>(D, A, wave, lane_again(), line2, base2, c2);
+  };
   if (odd) {  // the whole wavefront: its cells again, in plain divisions
-    int c2 = c;
-    asm volatile("" : "+v"(c2));  // read again, not kept from above
+    long line2, base2;
+    int c2;
+    again(line2, base2, c2);
     Cell q2;
-    if (TILE) q2 = tile_column<DIR, MAG>(D, A, c2, lds, c2 - c);
-    else q2 = load_cell<DIR, MAG, EXT>(D, A, base, line, c2);
-    line_faces_plain<DIR, MAG, LIM>(A, q2, c2 < -2 ? -2 : (c2 > n + 1 ? n + 1 : c2), gam,
-                                    gptr(D.sc)->ch, t, fe);
+    if (TILE) q2 = tile_column<DIR, MAG>(D, A, c2, lds);
+    else q2 = load_cell<DIR, MAG, EXT>(D, A, base2, line2, c2);
+    double fe[4];
+    line_faces_plain<DIR, MAG, LIM>(A, q2, c2, gam, gptr(D.sc)->ch, t, fe);
+    neg = fe[1] <= 0.0 || fe[0] <= 0.0 || fe[3] <= 0.0 || fe[2] <= 0.0;
   }
   const bool fxb = EXT && A.ext && flux_face(A, c);
   if (fxb) boundary_flux<DIR>(A, c, t);
+  lane = lane_again();
   // faces between lanes l and l+1 have valid slopes on both sides for l = 1..61
   const bool face_valid = valid && (c >= -1 && c <= n - 1) && lane >= 1 && lane <= 61 && !fxb;
-  if (face_valid && (fe[1] <= 0.0 || fe[0] <= 0.0 || fe[3] <= 0.0 || fe[2] <= 0.0)) {
-    int ii, jj, kk;
-    line_origin<DIR>(D, line, ii, jj, kk);
-    if (DIR == 0) ii = c; else if (DIR == 1) jj = c; else kk = c;
+  if (face_valid && neg) {
+    long line2, base2;
+    int ii, jj, kk, c2;
+    again(line2, base2, c2);
+    line_origin<DIR>(D, line2, ii, jj, kk);
+    if (DIR == 0) ii = c2; else if (DIR == 1) jj = c2; else kk = c2;
     atomicMin(&gptr(D.sc)->err, errkey(stage, 0, DIR + 1, ii, jj, kk, D));
   }
 
@@ -841,7 +909,9 @@ __device__ __forceinline__ void sweep_line(const Dev &D, long wave, int lane, in
   for (int s = 0; s < 9; ++s) tm[s] = up1(t[s]);
   // equation order: icnt imo1 imo2 imo3 iene img1 img2 img3 i9wv
   constexpr int a_ = DIR, b_ = (DIR + 1) % 3, c_ = (DIR + 2) % 3;
-  const double ix = gptr(A.idxi)[cc];
+  int ci = c;
+  asm volatile("" : "+v"(ci));  // one register until here, not c's 64-bit form
+  const double ix = gptr(A.idxi)[ci];
   double du[NVMAX];
   du[0] = ix * (tm[0] - t[0]);
   du[1 + a_] = ix * (tm[1] - t[1]);
@@ -853,11 +923,16 @@ __device__ __forceinline__ void sweep_line(const Dev &D, long wave, int lane, in
   du[5 + c_] = ix * (tm[7] - t[7]);
   du[8] = ix * (tm[8] - t[8]);
   if (FUSED) {
-    fused_rk<DIR, MAG, TILE>(D, A, base, c, lane, du, lds, stage, *rk, *dti, *cfm);
+    fused_rk<DIR, MAG, TILE>(D, A, (long)ubase, c, lane, du, lds, stage, *rk, *dti, *cfm);
     return;
   }
-  store_du<DIR, MAG, TILE>(D, A, base, c, lane, du, lds);
-  if (SPC) store_mass_flux<DIR>(D, line, c, lane, t[0]);
+  store_du<DIR, MAG, TILE>(D, A, (long)ubase, c, lane, du, lds);
+  if (SPC) {
+    long line2, base2;
+    int c2;
+    again(line2, base2, c2);
+    store_mass_flux<DIR>(D, line2, c2, lane, t[0]);
+  }
 }
 
 // One launch covers every solved direction: wavefronts [0, waves[0]) sweep
@@ -1439,17 +1514,21 @@ __device__ __forceinline__ void fused_rk(const Dev &D, const Axis &A, long base,
     }
     return;
   }
-  const int bw = blockDim.x >> 6, w = threadIdx.x >> 6;
+  // the tile addresses computed again: kept from the load they took registers
+  // the solver needs (9 spills)
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  const int bw = blockDim.x >> 6, w = t >> 6;
   const int ld = tile_ld(bw), fs = 64 * ld;
   __syncthreads();  // every wavefront has read its cells out of the tile
   {
-    double *p = lds + lane * ld + w;
+    double *p = lds + (t & 63) * ld + w;
 #pragma unroll
     for (int v = 0; v < NVMAX; ++v)
       if (v < nv) p[v * fs] = du[v];
   }
   __syncthreads();
-  const int t = threadIdx.x, r = t >> __builtin_ctz(bw), col = t & (bw - 1);
+  const int r = t >> __builtin_ctz(bw), col = t & (bw - 1);
   long m;
   if (tile_row_cell<MAG>(lds, bw, t, m)) {
     const double *p = lds + r * ld + col;
@@ -2055,6 +2134,9 @@ __device__ void kat_one(int which, long t, const double *in, double *out) {
       hlld_fast<true>(f, a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9], a[10], a[11],
                       a[12], a[13], a[14], a[15], a[16], a[17], a[18], a[19], a[20], a[21],
                       fden(a[22]), k);
+    // the sweep tests these on the way to the solver
+    for (int s : {8, 9, 10, 11, 22}) k.pos(a[s]);
+    for (int s : {2, 3, 4, 5, 6, 7, 14, 15, 16, 17, 18, 19}) k.num(a[s]);
     if (!FAST || k.bad())
       hlld(f, a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9], a[10], a[11], a[12],
            a[13], a[14], a[15], a[16], a[17], a[18], a[19], a[20], a[21], a[22]);
@@ -2065,6 +2147,8 @@ __device__ void kat_one(int which, long t, const double *in, double *out) {
     double c = 0.0;
     if (FAST) {
       k.pos(a[0]);
+      k.pos(a[1] * a[1]);
+      for (int s = 2; s < 5; ++s) k.num(a[s]);
       c = fast_cf(fden(a[0]), a[1], a[2], a[3], a[4], k);
     }
     if (!FAST || k.bad()) c = get_cf(a[0], a[1], a[2], a[3], a[4]);
@@ -2082,17 +2166,18 @@ __device__ void kat_one(int which, long t, const double *in, double *out) {
         G.Dp = fden(a[5] - a[4]);
         G.cf = (a[5] - a[4]) / (a[7] - a[4]);
         G.cb = (a[4] - a[3]) / (a[4] - a[6]);
-        r = fslope<LIM_MC>(a[0], a[1], a[2], G, k);
-        k.num((a[2] - a[1]) * G.Dp.b);  // in the sweep the right neighbour's test
+        r = fslope<LIM_MC>(a[0], a[1], a[2], G);
         k.pos(G.Dm.b);
         k.pos(G.Dp.b);
       } else {
         G.ida = a[3];
         G.idb = a[4];
         G.Dab = fden(a[3] + a[4]);
-        r = fslope<LIM_MINMOD>(a[0], a[1], a[2], G, k);
+        r = fslope<LIM_MINMOD>(a[0], a[1], a[2], G);
         k.pos(G.Dab.b);
       }
+      k.num(r);  // in the sweep a tiny slope is lost in its cell's value
+      for (int s = 0; s < 3; ++s) k.num(a[s]);
       // the sweep's slope may have a zero of the other sign: as q + h*S
       // (with q = 0) shows it
       bad = k.bad() || r == 0.0;

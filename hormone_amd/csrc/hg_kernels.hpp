@@ -61,6 +61,7 @@ struct Axis {
   const double2 *geo;
   int fast;
   int n;
+  unsigned n4_inv;   // floor(2^32 / (n + 4)), for lane_cell
   unsigned nlines;   // lines along this axis (ncell / n)
   unsigned nsub;     // lines laid end to end in one sweep sequence (lane_cell)
   long stride;       // element stride of this axis in the SoA arrays
@@ -82,6 +83,7 @@ enum { GF_D = 0, GF_P, GF_V1, GF_V2, GF_V3, GF_B1, GF_B2, GF_B3, GF_PHI, NGF };
 
 struct Dev {
   int n1, n2, n3;  // interior extents
+  unsigned n1_inv;  // floor(2^32 / n1), at most 2^32 - 1
   long ncell;
   int nv, nw;      // conserved / primitive field counts
   int mag, dim, limiter;

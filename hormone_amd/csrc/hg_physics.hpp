@@ -281,22 +281,35 @@ __device__ __forceinline__ void hlld(R f[9], R cfl, R cfr, R v1l, R v1r, R v2l, 
 // (cell_slopes, face_flux).  One test per face instead of a branch per
 // division leaves the compiler one straight block to schedule.  The y and z
 // sweeps are bound by VALU issue (about 85% busy), so this is their time:
-// 1,530 -> 1,288 VALU instructions per wavefront (256^3 MHD shear layer),
-// 2,075 -> 1,893 us per stage for both; hydro (160^3, three directions in one
+// 1,530 -> 1,124 VALU instructions per wavefront (256^3 MHD shear layer),
+// 2,075 -> 1,760 us per stage for both; hydro (160^3, three directions in one
 // launch) 594 -> 437 us.
 //
 // Chk: pos() takes a value that has to be positive with an exponent in
-// [-256, 255]; num() one that may also be zero (its frexp exponent is 0 then,
-// as it is for NaN and infinities, whose quotients v_div_fixup returns
-// without reading the reciprocal).  With both in range a quotient lies in
-// 2^+-512, far from the exponents v_div_scale acts on (a denormal or inexact
-// residual needs a dividend below 2^-968, an extreme quotient exponents more
-// than 768 apart).
+// [-256, 255], neg() a negative one, num() one of either sign that may also be
+// zero (its frexp exponent is 0 then), differ() a pair whose order decides.
+//
+// What is tested, and why it is enough.  A quotient or root without scaling is
+// exact unless its dividend or radicand is below 2^-968 (an inexact residual),
+// the divisor extreme, or the quotient overflows or is denormal.
+// * Every cell (odd_cell): d, e and e_int in range, so |m| <= 2^257 and |b| <=
+//   2^129; no NaN, infinity or -0.  Face densities and energies, the squared
+//   sound speeds, and every divisor and radicand of the solver: in range.  So
+//   no divisor is extreme and no quotient overflows.
+// * What is left are dividends that are tiny but not zero.  Their quotients are
+//   tiny too and wrong by an ulp at most.  Such a value is lost in a sum with
+//   any value in range, and the sums that always hold one need no test: the
+//   energies and pressures, the wave speeds (a fast speed is in range), pta.
+//   Where all of a sum may be tiny its result is tested: sm's dividend, b1,
+//   the face's psi and, for all that feeds them (the limited slopes, the
+//   velocities, the star states), the selected transverse velocity and field.
 // The tests are asm volatile so that each is made where its value is computed:
 // written as expressions they were gathered at the end of the block, with
-// every tested value kept in registers until then (162 instead of 126 VGPRs).
+// every tested value kept in registers until then (162 VGPRs against 126; 102
+// with the fluxes forced before the branch, see line_faces).
 struct Chk {
   unsigned n = 0, p = 0;
+  bool near = false;
   __device__ __forceinline__ void num(double x) {
     unsigned t;
     asm volatile(
@@ -306,7 +319,11 @@ struct Chk {
   }
   __device__ __forceinline__ void pos(double x) { high<0xd0100000u>(__double2hiint(x)); }
   __device__ __forceinline__ void neg(double x) { high<0x50100000u>(__double2hiint(x)); }
-  __device__ __forceinline__ bool bad() const { return (n & ~511u) || (p & 0xe0000000u); }
+  // d = x - y, y >= 0: false (0 - 0 apart) within 2^-48 of y
+  __device__ __forceinline__ void differ(double d, double y) { near |= fabs(d) < 0x1p-48 * y; }
+  __device__ __forceinline__ bool bad() const {
+    return (n & ~511u) || (p & 0xe0000000u) || near;
+  }
 
  private:
   template <unsigned MINUS>  // -(high word of the smallest value in range)
@@ -380,24 +397,18 @@ struct Geo {
 // that only move a sign taken out: sig*0.5*(bot+top) = flip(0.5*(bot+top)),
 // sig*cf*bot = cf*|bot|, sig*cb*top = flip(cb*top) (rounding is symmetric).
 template <int LIM>
-__device__ __forceinline__ double fslope(double u0, double u1, double u2, const Geo &G, Chk &k) {
+__device__ __forceinline__ double fslope(double u0, double u1, double u2, const Geo &G) {
   if constexpr (LIM == LIM_MINMOD) {
     const double x = 1.4 * (u2 - u1) * G.idb;
     const double y = 1.4 * (u1 - u0) * G.ida;
-    const double zn = (u2 - u0) * G.ida * G.idb;
-    k.num(zn);
     const unsigned s = sbit(x);
-    const double z = fdiv_(G.Dab, zn);
+    const double z = fdiv_(G.Dab, (u2 - u0) * G.ida * G.idb);
     return flip(vmax0(vmin(vmin(fabs(x), flip(y, s)), flip(z, s))), s);
   } else {
-    const double tn = (u1 - u0) * G.Dp.b;
-    k.num(tn);
-    const double top = fdiv_(G.Dm, tn);
+    const double top = fdiv_(G.Dm, (u1 - u0) * G.Dp.b);
     const double bot = u2 - u1;
     const unsigned s = sbit(bot);
     const double m = vmin(vmin(flip(0.5 * (bot + top), s), G.cf * fabs(bot)), flip(G.cb * top, s));
-    // its dividend needs no test: 0 or at least half the smaller of |bot| and
-    // |top|, top in range with tn, bot with the right neighbour's tn
     return fdiv_(G.Dp, flip(vmax0(m), s));
   }
 }
@@ -408,9 +419,8 @@ __device__ __forceinline__ double fslope(double u0, double u1, double u2, const 
 // guard's own face values are the Riemann states unless it resets the slopes
 // to zero (then they are the cell's value), so nothing is evaluated twice.
 //
-// A cell with a NaN, an infinity or a -0 is sent to the plain path: vmin and
-// vmax treat those otherwise than the reference's comparisons.  With none of
-// them a slope's zero may have the other sign, which q +- h*S does not show.
+// odd_cell keeps out what vmin and vmax treat otherwise; a slope's zero may
+// have the other sign, which q +- h*S does not show where q is not -0.
 template <bool MAG, int LIM>
 __device__ __forceinline__ void cell_faces(const double qv[9], const double ql[9],
                                            const double qr[9], const Geo &G, double FL[8],
@@ -419,7 +429,6 @@ __device__ __forceinline__ void cell_faces(const double qv[9], const double ql[9
   if constexpr (LIM == LIM_FLAT) {
 #pragma unroll
     for (int s = 0; s < 8; ++s) FL[s] = FR[s] = s < NS ? qv[s] : 0.0;
-    k.pos(qv[0]);
     DL = DR = fden(qv[0]);
     return;
   }
@@ -429,7 +438,7 @@ __device__ __forceinline__ void cell_faces(const double qv[9], const double ql[9
       FL[s] = FR[s] = 0.0;
       continue;
     }
-    const double S = fslope<LIM>(ql[s], qv[s], qr[s], G, k);
+    const double S = fslope<LIM>(ql[s], qv[s], qr[s], G);
     FL[s] = qv[s] - G.hl * S;
     FR[s] = qv[s] + G.hr * S;
     if (s % 4 == 3) fence();
@@ -437,12 +446,12 @@ __device__ __forceinline__ void cell_faces(const double qv[9], const double ql[9
   fence();
   k.pos(FL[0]);
   k.pos(FR[0]);
+  k.pos(FL[1]);
+  k.pos(FR[1]);
   DL = fden(FL[0]);
   DR = fden(FR[0]);
   const double kl = 0.5 * (FL[2] * FL[2] + FL[3] * FL[3] + FL[4] * FL[4]);
   const double kr = 0.5 * (FR[2] * FR[2] + FR[3] * FR[3] + FR[4] * FR[4]);
-  k.num(kl);
-  k.num(kr);
   double eintl = FL[1] - fdiv_(DL, kl);
   double eintr = FR[1] - fdiv_(DR, kr);
   if (MAG) {
@@ -454,27 +463,29 @@ __device__ __forceinline__ void cell_faces(const double qv[9], const double ql[9
       eintr <= vmin(em_, er_)) {
 #pragma unroll
     for (int s = 0; s < NS; ++s) FL[s] = FR[s] = qv[s];
-    k.pos(qv[0]);
     DL = DR = fden(qv[0]);
   }
 }
 
-// cell values vmin and vmax may not see (NaN, infinity, -0)
+// A cell the fast form is not for: d, e or e_int out of range, or a momentum or
+// field that is NaN, infinite or -0 (vmin and vmax treat those otherwise than
+// the reference's comparisons).
 template <bool MAG>
 __device__ __forceinline__ bool odd_cell(const double qv[9]) {
-  bool b = __builtin_amdgcn_class(qv[8], 0x227);
+  Chk k;
+  k.pos(qv[0]);
+  k.pos(qv[1]);
+  k.pos(qv[8]);
+  bool b = k.bad();
 #pragma unroll
-  for (int s = 0; s < (MAG ? 8 : 5); ++s) b |= __builtin_amdgcn_class(qv[s], 0x227);
+  for (int s = 2; s < (MAG ? 8 : 5); ++s) b |= __builtin_amdgcn_class(qv[s], 0x227);
   return b;
 }
 
-// get_cf, the checked fast form; asq = cs*cs is in range (the caller's pos()),
-// so a quotient b*b/d too small for fdiv_ is lost in the sum as it is in the
-// reference's, and one too large shows in the radicand
+// get_cf, the checked fast form
 __device__ __forceinline__ double fast_cf(const Den64 &Dd, double cs, double b1, double b2,
                                           double b3, Chk &k) {
   const double asq = cs * cs;
-  k.pos(asq);
   const double bb1 = fdiv_(Dd, b1 * b1);
   const double bb2 = fdiv_(Dd, b2 * b2);
   const double bb3 = fdiv_(Dd, b3 * b3);
@@ -497,6 +508,17 @@ __device__ __forceinline__ void hlld_fast(double f[9], double cfl, double cfr, d
                                           double ptl, double ptr, double b1l, double b1r,
                                           double b2l, double b2r, double b3l, double b3r,
                                           double phil, double phir, const Den64 &Dch, Chk &k) {
+  double b1 = 0.0, phi = 0.0;
+  const double ch = Dch.b;
+  if constexpr (MAG) {  // first: psi and the sides' normal fields are done with then
+    const double dphi = phir - phil;
+    k.num(dphi);
+    b1 = 0.5 * ((b1l + b1r) - fdiv_(Dch, dphi));
+    phi = 0.5 * ((phil + phir) - (b1r - b1l) * ch);
+    k.num(b1);
+    k.num(phi);
+    fence();
+  }
   const double sl = vmin(vmin(v1r - cfr, v1l - cfl), 0.0);
   const double sr = vmax(vmax(v1r + cfr, v1l + cfl), 0.0);
   const double slv = sl - v1l, srv = sr - v1r;
@@ -506,7 +528,6 @@ __device__ __forceinline__ void hlld_fast(double f[9], double cfl, double cfr, d
   const double smn = srv * dr * v1r - slv * dl * v1l - ptr + ptl;
   const double pan = srv * dr * ptl - slv * dl * ptr + dl * dr * srv * slv * (v1r - v1l);
   k.num(smn);
-  k.num(pan);
   const double sm = fdiv_(Dden, smn), pta = fdiv_(Dden, pan);
   const double slm = sl - sm, srm = sr - sm;
   k.neg(slm);
@@ -518,69 +539,63 @@ __device__ __forceinline__ void hlld_fast(double f[9], double cfl, double cfr, d
   fence();
   const int hsm = __double2hiint(sm);
   if constexpr (!MAG) {
-    const double eln = slv * el - ptl * v1l + pta * sm, ern = srv * er - ptr * v1r + pta * sm;
-    k.num(eln);
-    k.num(ern);
-    const double ela = fdiv_(Dslm, eln), era = fdiv_(Dsrm, ern);
+    const double ela = fdiv_(Dslm, slv * el - ptl * v1l + pta * sm);
+    const double era = fdiv_(Dsrm, srv * er - ptr * v1r + pta * sm);
     const double wl = wpos(hsm), wr = wneg(hsm);
     const double d_ = wl * dla + wr * dra;
+    const double v2_ = wl * v2l + wr * v2r, v3_ = wl * v3l + wr * v3r;
+    k.num(v2_);
+    k.num(v3_);
     f[0] = d_ * sm;
     f[1] = d_ * sm * sm + pta;
-    f[2] = d_ * sm * (wl * v2l + wr * v2r);
-    f[3] = d_ * sm * (wl * v3l + wr * v3r);
+    f[2] = d_ * sm * v2_;
+    f[3] = d_ * sm * v3_;
     f[4] = ((wl * ela + wr * era) + pta) * sm;
     f[5] = f[6] = f[7] = f[8] = 0.0;
     return;
   }
-  const double ch = Dch.b;
-  const double dphi = phir - phil;
-  k.num(dphi);
-  k.pos(ch);
-  const double b1 = 0.5 * ((b1l + b1r) - fdiv_(Dch, dphi));
-  const double phi = 0.5 * ((phil + phir) - (b1r - b1l) * ch);
-
   const double sqla = fsqrt(dla), sqra = fsqrt(dra);
+  // the Alfven speeds sm -+ |b1|/sqrt(rho) only select by their sign: that of
+  // sm*sqrt(rho) -+ |b1|, unless the two nearly cancel
   const double ab1 = fabs(b1);
-  k.num(b1);
-  const double sla = sm - fdiv_(fden(sqla), ab1);
-  const double sra = sm + fdiv_(fden(sqra), ab1);
-
-  const double b1b1 = b1 * b1;
-  const double dnl = dl * slv * slm - b1b1, dnr = dr * srv * srm - b1b1;
-  k.pos(dnl);
-  k.pos(dnr);
-  const Den64 Dl = fden(dnl), Dr = fden(dnr);
-  auto qd = [&](const Den64 &D, double a) {
-    k.num(a);
-    return fdiv_(D, a);
-  };
-  const double v2la = v2l - qd(Dl, b1 * b2l * (sm - v1l));
-  const double v2ra = v2r - qd(Dr, b1 * b2r * (sm - v1r));
-  const double v3la = v3l - qd(Dl, b1 * b3l * (sm - v1l));
-  const double v3ra = v3r - qd(Dr, b1 * b3r * (sm - v1r));
-  const double numl = dl * slv * slv - b1b1;
-  const double numr = dr * srv * srv - b1b1;
-  const double b2la = qd(Dl, b2l * numl);
-  const double b2ra = qd(Dr, b2r * numr);
-  const double b3la = qd(Dl, b3l * numl);
-  const double b3ra = qd(Dr, b3r * numr);
+  const double sla = fma(sm, sqla, -ab1), sra = fma(sm, sqra, ab1);
+  k.differ(sla, ab1);
+  k.differ(sra, ab1);
   fence();
 
-  const double ela = qd(Dslm, slv * el - ptl * v1l + pta * sm +
-                                  b1 * ((v1l * b1 + v2l * b2l + v3l * b3l) -
-                                        (sm * b1 + v2la * b2la + v3la * b3la)));
-  const double era = qd(Dsrm, srv * er - ptr * v1r + pta * sm +
-                                  b1 * ((v1r * b1 + v2r * b2r + v3r * b3r) -
-                                        (sm * b1 + v2ra * b2ra + v3ra * b3ra)));
-
+  const double b1b1 = b1 * b1;
+  // one side after the other: a side's face values are done with then
+  const double dnl = dl * slv * slm - b1b1;
+  k.pos(dnl);
+  const Den64 Dl = fden(dnl);
+  const double v2la = v2l - fdiv_(Dl, b1 * b2l * (sm - v1l));
+  const double v3la = v3l - fdiv_(Dl, b1 * b3l * (sm - v1l));
+  const double numl = dl * slv * slv - b1b1;
+  const double b2la = fdiv_(Dl, b2l * numl);
+  const double b3la = fdiv_(Dl, b3l * numl);
+  const double ela = fdiv_(Dslm, slv * el - ptl * v1l + pta * sm +
+                                     b1 * ((v1l * b1 + v2l * b2l + v3l * b3l) -
+                                           (sm * b1 + v2la * b2la + v3la * b3la)));
+  fence();
+  const double dnr = dr * srv * srm - b1b1;
+  k.pos(dnr);
+  const Den64 Dr = fden(dnr);
+  const double v2ra = v2r - fdiv_(Dr, b1 * b2r * (sm - v1r));
+  const double v3ra = v3r - fdiv_(Dr, b1 * b3r * (sm - v1r));
+  const double numr = dr * srv * srv - b1b1;
+  const double b2ra = fdiv_(Dr, b2r * numr);
+  const double b3ra = fdiv_(Dr, b3r * numr);
+  const double era = fdiv_(Dsrm, srv * er - ptr * v1r + pta * sm +
+                                     b1 * ((v1r * b1 + v2r * b2r + v3r * b3r) -
+                                           (sm * b1 + v2ra * b2ra + v3ra * b3ra)));
   fence();
   const unsigned s1 = sbit(b1);
   const Den64 Dsqs = fden(sqla + sqra);
-  const double v2aa = qd(Dsqs, sqla * v2la + sqra * v2ra + flip(b2ra - b2la, s1));
-  const double v3aa = qd(Dsqs, sqla * v3la + sqra * v3ra + flip(b3ra - b3la, s1));
+  const double v2aa = fdiv_(Dsqs, sqla * v2la + sqra * v2ra + flip(b2ra - b2la, s1));
+  const double v3aa = fdiv_(Dsqs, sqla * v3la + sqra * v3ra + flip(b3ra - b3la, s1));
   const double sqp = fsqrt(dla * dra);
-  const double b2aa = qd(Dsqs, sqla * b2ra + sqra * b2la + flip(sqp * (v2ra - v2la), s1));
-  const double b3aa = qd(Dsqs, sqla * b3ra + sqra * b3la + flip(sqp * (v3ra - v3la), s1));
+  const double b2aa = fdiv_(Dsqs, sqla * b2ra + sqra * b2la + flip(sqp * (v2ra - v2la), s1));
+  const double b3aa = fdiv_(Dsqs, sqla * b3ra + sqra * b3la + flip(sqp * (v3ra - v3la), s1));
 
   fence();
   const double vbaa = v2aa * b2aa + v3aa * b3aa;
@@ -594,6 +609,10 @@ __device__ __forceinline__ void hlld_fast(double f[9], double cfl, double cfr, d
   const double v3_ = wl * v3la + wa * v3aa + wr * v3ra;
   const double b2_ = wl * b2la + wa * b2aa + wr * b2ra;
   const double b3_ = wl * b3la + wa * b3aa + wr * b3ra;
+  k.num(v2_);
+  k.num(v3_);
+  k.num(b2_);
+  k.num(b3_);
   const double e_ = wl * ela + wneg(hla ^ hsm) * elaa + wneg(hsm ^ hra) * eraa + wr * era;
   f[0] = d_ * sm;
   f[1] = d_ * sm * sm + pta - b1b1;
@@ -607,53 +626,41 @@ __device__ __forceinline__ void hlld_fast(double f[9], double cfl, double cfr, d
 }
 
 // Face states to flux, as face_flux: L the left cell's FR, R_ the right
-// cell's FL, Dl and Dr their densities' reciprocals; fe: dl eil dr eir.
+// cell's FL, Dl and Dr their densities' reciprocals.  A face density or
+// internal energy that is not positive fails its test (pos), so the
+// reference's stop on it is left to the plain form.
 template <int DIR, bool MAG>
 __device__ __forceinline__ void face_fast(const double L[8], const double R_[8], double phil,
                                           double phir, const Den64 &Dl, const Den64 &Dr,
-                                          double gam, const Den64 &Dch, double t[9], double fe[4],
-                                          Chk &k) {
+                                          double gam, const Den64 &Dch, double t[9], Chk &k) {
   constexpr int a_ = DIR, b_ = (DIR + 1) % 3, c_ = (DIR + 2) % 3;
-  auto qd = [&](const Den64 &D, double a) {
-    k.num(a);
-    return fdiv_(D, a);
+  struct Side {
+    double v1, v2, v3, b1, b2, b3, pt, cf;
   };
-  const double v1l = qd(Dl, L[2 + a_]), v1r = qd(Dr, R_[2 + a_]);
-  const double v2l = qd(Dl, L[2 + b_]), v2r = qd(Dr, R_[2 + b_]);
-  const double v3l = qd(Dl, L[2 + c_]), v3r = qd(Dr, R_[2 + c_]);
-  double b1l = 0, b1r = 0, b2l = 0, b2r = 0, b3l = 0, b3r = 0;
-  if (MAG) {
-    b1l = L[5 + a_];
-    b1r = R_[5 + a_];
-    b2l = L[5 + b_];
-    b2r = R_[5 + b_];
-    b3l = L[5 + c_];
-    b3r = R_[5 + c_];
-  }
-  const double eil = get_eint(MAG, L[1], L[0], v1l, v2l, v3l, b1l, b2l, b3l);
-  const double eir = get_eint(MAG, R_[1], R_[0], v1r, v2r, v3r, b1r, b2r, b3r);
-  fe[0] = L[0];
-  fe[1] = eil;
-  fe[2] = R_[0];
-  fe[3] = eir;
-  fence();
-  double ptl = (gam - 1.0) * eil, ptr = (gam - 1.0) * eir;
-  // quotients in range (pos) with the density in range: so was the dividend
-  const double asl = fdiv_(Dl, gam * ptl), asr = fdiv_(Dr, gam * ptr);
-  k.pos(asl);
-  k.pos(asr);
-  double cfl = fsqrt(asl), cfr = fsqrt(asr);
-  if (MAG) {
-    ptl = ptl + 0.5 * (b1l * b1l + b2l * b2l + b3l * b3l);
-    ptr = ptr + 0.5 * (b1r * b1r + b2r * b2r + b3r * b3r);
-    cfl = fast_cf(Dl, cfl, b1l, b2l, b3l, k);
-    cfr = fast_cf(Dr, cfr, b1r, b2r, b3r, k);
-  }
-  fence();
+  auto side = [&](const double F[8], const Den64 &Df) {
+    Side o;
+    o.v1 = fdiv_(Df, F[2 + a_]);
+    o.v2 = fdiv_(Df, F[2 + b_]);
+    o.v3 = fdiv_(Df, F[2 + c_]);
+    o.b1 = MAG ? F[5 + a_] : 0.0;
+    o.b2 = MAG ? F[5 + b_] : 0.0;
+    o.b3 = MAG ? F[5 + c_] : 0.0;
+    o.pt = (gam - 1.0) * get_eint(MAG, F[1], F[0], o.v1, o.v2, o.v3, o.b1, o.b2, o.b3);
+    const double as = fdiv_(Df, gam * o.pt);
+    k.pos(as);
+    o.cf = fsqrt(as);
+    if (MAG) {
+      o.pt = o.pt + 0.5 * (o.b1 * o.b1 + o.b2 * o.b2 + o.b3 * o.b3);
+      o.cf = fast_cf(Df, o.cf, o.b1, o.b2, o.b3, k);
+    }
+    fence();  // one side after the other, for the registers
+    return o;
+  };
+  const Side l = side(L, Dl), r = side(R_, Dr);
   // without B get_cf is sqrt(0.5*(cs^2 + sqrt(cs^4))) = cs exactly: the
   // square root of a rounded square is the number itself
-  hlld_fast<MAG>(t, cfl, cfr, v1l, v1r, v2l, v2r, v3l, v3r, L[0], R_[0], L[1], R_[1], ptl, ptr,
-                 b1l, b1r, b2l, b2r, b3l, b3r, phil, phir, Dch, k);
+  hlld_fast<MAG>(t, l.cf, r.cf, l.v1, r.v1, l.v2, r.v2, l.v3, r.v3, L[0], R_[0], L[1], R_[1],
+                 l.pt, r.pt, l.b1, r.b1, l.b2, r.b2, l.b3, r.b3, phil, phir, Dch, k);
 }
 
 // ---- FP32-mixed HLLD in perturbation form ----------------------------------
