@@ -1192,8 +1192,18 @@ __global__ __launch_bounds__(1024) void k_sweep_mix(Dev D, int stage) {
 // second fetch by another XCD.  Measured on the 256^3 MHD polytrope: y+z
 // sweep 2244 -> 2052 us; the same renumbering of the streaming x blocks (the
 // fused x sweep) and of the gravity sub-steps made them 3-6% slower.
-template <int DIR, bool MAG, int LIM, bool TILE, bool MIX>
-__global__ __launch_bounds__(1024) void k_sweep_dir(Dev D, int stage) {
+//
+// TH: the most threads a block has.  Blocks of up to SMALL_BLOCK threads run
+// the instantiation held to 96 VGPRs: five waves per SIMD (five 29.7 KB MHD
+// tiles fit the 160 KB of LDS) instead of four, without a spill outside the
+// rarely run plain division path.  256^3 MHD: y+z 1695 -> 1649 us (polytrope)
+// and 1759 -> 1733 us (shear); fused x sweep of 512^2 24.2 -> 21.7 us.  Larger
+// blocks need 1024-thread bounds, and k_sweep, which holds three directions,
+// would spill in every one of them (128^2: 11.3 -> 13.5 us).
+constexpr int SMALL_BLOCK = 256, LARGE_BLOCK = 1024;
+
+template <int DIR, bool MAG, int LIM, bool TILE, bool MIX, int TH>
+__global__ __launch_bounds__(TH, TH == SMALL_BLOCK ? 5 : 4) void k_sweep_dir(Dev D, int stage) {
   extern __shared__ double lds[];
   if (gptr(D.sc)->stop) return;
   const int lane = threadIdx.x & 63;
@@ -1541,9 +1551,9 @@ __device__ __forceinline__ void fused_rk(const Dev &D, const Axis &A, long base,
 }
 
 // One wavefront per segment of a DIR line, as k_sweep; CFL partials (last
-// stage) one per block.
-template <int DIR, bool MAG, int LIM, bool TILE, bool MIX = false>
-__global__ __launch_bounds__(1024) void k_sweep_rk(Dev D, int stage, RKArgs rk) {
+// stage) one per block.  TH as k_sweep_dir.
+template <int DIR, bool MAG, int LIM, bool TILE, bool MIX, int TH>
+__global__ __launch_bounds__(TH, TH == SMALL_BLOCK ? 5 : 4) void k_sweep_rk(Dev D, int stage, RKArgs rk) {
   extern __shared__ double lds[];
   if (gptr(D.sc)->stop) return;
   const int lane = threadIdx.x & 63;
@@ -2362,49 +2372,63 @@ void launch_species(const Dev &D, hipStream_t s) {
   else klaunch(k_species<LIM_MC>, g, 256, s, nullptr, D);
 }
 
-template <int DIR, bool MAG, int LIM>
+template <int DIR, bool MAG, int LIM, int TH>
 static void sweep_rk_variant(const Dev &D, int stage, const RKArgs &rk, unsigned g, int bs,
                              size_t tile, hipStream_t s, const KEv *ev) {
   if constexpr (DIR > 0) {  // x lines are lane lines, never tiled
     if (tile) {
-      if (D.mixed) klaunch_lds(k_sweep_rk<DIR, MAG, LIM, true, true>, g, bs, tile, s, ev, D, stage, rk);
-      else klaunch_lds(k_sweep_rk<DIR, MAG, LIM, true>, g, bs, tile, s, ev, D, stage, rk);
+      if (D.mixed) klaunch_lds(k_sweep_rk<DIR, MAG, LIM, true, true, TH>, g, bs, tile, s, ev, D, stage, rk);
+      else klaunch_lds(k_sweep_rk<DIR, MAG, LIM, true, false, TH>, g, bs, tile, s, ev, D, stage, rk);
       return;
     }
   }
   // the lane path parks each thread's primitives (park_cell)
   const size_t park = (size_t)park_fields(MAG) * sizeof(double) * (size_t)bs;
-  if (D.mixed) klaunch_lds(k_sweep_rk<DIR, MAG, LIM, false, true>, g, bs, park, s, ev, D, stage, rk);
-  else klaunch_lds(k_sweep_rk<DIR, MAG, LIM, false>, g, bs, park, s, ev, D, stage, rk);
+  if (D.mixed) klaunch_lds(k_sweep_rk<DIR, MAG, LIM, false, true, TH>, g, bs, park, s, ev, D, stage, rk);
+  else klaunch_lds(k_sweep_rk<DIR, MAG, LIM, false, false, TH>, g, bs, park, s, ev, D, stage, rk);
+}
+
+template <int DIR, int TH>
+static void sweep_rk_dir_th(const Dev &D, int stage, const RKArgs &rk, unsigned g, int bs,
+                            size_t tile, hipStream_t s, const KEv *ev) {
+  if (D.mag) {
+    if (D.limiter == LIM_FLAT) sweep_rk_variant<DIR, true, LIM_FLAT, TH>(D, stage, rk, g, bs, tile, s, ev);
+    else if (D.limiter == LIM_MINMOD) sweep_rk_variant<DIR, true, LIM_MINMOD, TH>(D, stage, rk, g, bs, tile, s, ev);
+    else sweep_rk_variant<DIR, true, LIM_MC, TH>(D, stage, rk, g, bs, tile, s, ev);
+  } else {
+    if (D.limiter == LIM_FLAT) sweep_rk_variant<DIR, false, LIM_FLAT, TH>(D, stage, rk, g, bs, tile, s, ev);
+    else if (D.limiter == LIM_MINMOD) sweep_rk_variant<DIR, false, LIM_MINMOD, TH>(D, stage, rk, g, bs, tile, s, ev);
+    else sweep_rk_variant<DIR, false, LIM_MC, TH>(D, stage, rk, g, bs, tile, s, ev);
+  }
 }
 
 template <int DIR>
 static void sweep_rk_dir(const Dev &D, int stage, const RKArgs &rk, unsigned g, int bs,
                          size_t tile, hipStream_t s, const KEv *ev) {
-  if (D.mag) {
-    if (D.limiter == LIM_FLAT) sweep_rk_variant<DIR, true, LIM_FLAT>(D, stage, rk, g, bs, tile, s, ev);
-    else if (D.limiter == LIM_MINMOD) sweep_rk_variant<DIR, true, LIM_MINMOD>(D, stage, rk, g, bs, tile, s, ev);
-    else sweep_rk_variant<DIR, true, LIM_MC>(D, stage, rk, g, bs, tile, s, ev);
+  if (bs <= SMALL_BLOCK) sweep_rk_dir_th<DIR, SMALL_BLOCK>(D, stage, rk, g, bs, tile, s, ev);
+  else sweep_rk_dir_th<DIR, LARGE_BLOCK>(D, stage, rk, g, bs, tile, s, ev);
+}
+
+template <int DIR, bool MAG, int LIM, int TH>
+static void sweep_dir_th(const Dev &D, int stage, int bs, size_t tile, hipStream_t s,
+                         const KEv *ev) {
+  const unsigned g = nblk(D.waves[DIR], bs / 64);
+  const bool t = DIR > 0 && tile;
+  if (D.mixed) {
+    if (t) klaunch_lds(k_sweep_dir<DIR, MAG, LIM, true, true, TH>, g, bs, tile, s, ev, D, stage);
+    else klaunch_lds(k_sweep_dir<DIR, MAG, LIM, false, true, TH>, g, bs, 0, s, ev, D, stage);
   } else {
-    if (D.limiter == LIM_FLAT) sweep_rk_variant<DIR, false, LIM_FLAT>(D, stage, rk, g, bs, tile, s, ev);
-    else if (D.limiter == LIM_MINMOD) sweep_rk_variant<DIR, false, LIM_MINMOD>(D, stage, rk, g, bs, tile, s, ev);
-    else sweep_rk_variant<DIR, false, LIM_MC>(D, stage, rk, g, bs, tile, s, ev);
+    if (t) klaunch_lds(k_sweep_dir<DIR, MAG, LIM, true, false, TH>, g, bs, tile, s, ev, D, stage);
+    else klaunch_lds(k_sweep_dir<DIR, MAG, LIM, false, false, TH>, g, bs, 0, s, ev, D, stage);
   }
 }
 
 template <int DIR, bool MAG, int LIM>
 static void sweep_dir_launch(const Dev &D, int stage, int bw, size_t tile, hipStream_t s,
                              const KEv *ev) {
-  const unsigned g = nblk(D.waves[DIR], bw);
   const int bs = 64 * bw;
-  const bool t = DIR > 0 && tile;
-  if (D.mixed) {
-    if (t) klaunch_lds(k_sweep_dir<DIR, MAG, LIM, true, true>, g, bs, tile, s, ev, D, stage);
-    else klaunch_lds(k_sweep_dir<DIR, MAG, LIM, false, true>, g, bs, 0, s, ev, D, stage);
-  } else {
-    if (t) klaunch_lds(k_sweep_dir<DIR, MAG, LIM, true, false>, g, bs, tile, s, ev, D, stage);
-    else klaunch_lds(k_sweep_dir<DIR, MAG, LIM, false, false>, g, bs, 0, s, ev, D, stage);
-  }
+  if (bs <= SMALL_BLOCK) sweep_dir_th<DIR, MAG, LIM, SMALL_BLOCK>(D, stage, bs, tile, s, ev);
+  else sweep_dir_th<DIR, MAG, LIM, LARGE_BLOCK>(D, stage, bs, tile, s, ev);
 }
 
 template <bool MAG, int LIM>
