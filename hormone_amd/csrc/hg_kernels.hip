@@ -1310,7 +1310,7 @@ __device__ __forceinline__ void cfl_cell(const Dev &D, long m, double d, double 
     cf2 = cs + fabs(v2);
     cf3 = cs + fabs(v3);
   }
-  const double x1 = D.ax[0].dxi[i], x2 = D.ax[1].dxi[j], x3 = D.ax[2].dxi[k];
+  const double x1 = gptr(D.ax[0].dxi)[i], x2 = gptr(D.ax[1].dxi)[j], x3 = gptr(D.ax[2].dxi)[k];
   const double dvol = x1 * x2 * x3;  // metric.f90:44-47
   const double sa1 = x2 * x3, sa2 = x1 * x3, sa3 = x1 * x2;
   const double o1 = D.solve[0] ? 1.0 : 0.0, o2 = D.solve[1] ? 1.0 : 0.0,
@@ -1367,7 +1367,7 @@ __device__ __forceinline__ void grav_source(const Dev &D, long m, double src[NVM
                                             const Cell *qc = nullptr) {
   int i, j, k;
   cell_ijk(D, m, i, j, k);
-  const double *ph = D.gphi[D.gcur];
+  const auto ph = gptr(D.gphi[D.gcur]);
   const long g = gidx(D, i, j, k);
   const long st[3] = {1, (long)(D.n1 + 2), (long)(D.n1 + 2) * (D.n2 + 2)};
   const int q3[3] = {i, j, k};
@@ -1376,7 +1376,7 @@ __device__ __forceinline__ void grav_source(const Dev &D, long m, double src[NVM
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
     const int q = q3[a];
-    const double *DX = D.ax[a].dx, *IDX = D.ax[a].idx;
+    const auto DX = gptr(D.ax[a].dx), IDX = gptr(D.ax[a].idx);
     gr[a] = -((DX[q] * IDX[q + 1] * ph[g + st[a]] - DX[q + 1] * IDX[q] * ph[g - st[a]]) /
                   (DX[q] + DX[q + 1]) +
               (DX[q + 1] - DX[q]) * IDX[q] * IDX[q + 1] * ph[g]) *
@@ -1394,71 +1394,114 @@ __device__ __forceinline__ void grav_source(const Dev &D, long m, double src[NVM
 // LD >= 0: direction LD's flux divergence comes from duL[] (the fused last
 // sweep) instead of memory.  The flags are plain arguments so that one
 // inlined copy serves every variant; k_rk passes constants.
-// qc: the cell's current primitives (parked_cell) when the caller holds
+// park: the cell's current primitives (park_cell) when the caller has parked
 // them: d, e and B are then not read from U again.
-template <bool MAG, int LD = -1>
+template <bool MAG, int LD = -1, bool PARK = false>
 __device__ __forceinline__ void rk_cell_rt(const Dev &D, long m, int stage, double faco,
                                            double fact, double facn, double damp, bool CFL,
                                            bool DAMP, bool GRAV, double &dti, double &cfm,
                                            const double *duL = nullptr,
-                                           const Cell *qc = nullptr) {
+                                           const double *park = nullptr) {
   // the fused form writes the new state to the other buffer set (the
   // launch's neighbours still read this one); k_rk updates in place
   double *const *Uo = LD >= 0 ? D.Uo : D.U;
   double *const *Wo = LD >= 0 ? D.Wo : D.W;
-  const double ft = fact * gptr(D.sc)->dt;
-  double src[NVMAX];
-  if (GRAV) grav_source(D, m, src, qc);
-  double un[NVMAX];
-  double dold = 0.0;  // stage-start density (primitive d = u(icnt))
-  // a bound known at compile time for hydro, so that the loop unrolls and
-  // un[] stays in registers
-  const int nv = MAG ? D.nv : 5;
+  // Everything the update reads is loaded before anything is stored: the
+  // stores might alias, and a load written after one waits for it, nine memory
+  // round trips in a row (@R@).  Two groups, the divergences and the states, as
+  // many as registers allow in flight; a psi that is not there reads B3 again,
+  // so that each group is straight code.
+  const bool psi = MAG && D.nv == 9;
+  constexpr int nv = MAG ? 9 : 5;
+  auto load = [&](double *const *F, double x[NVMAX]) {
+    double *const last = psi ? F[8] : F[7];
+#pragma unroll
+    for (int v = 0; v < nv; ++v) x[v] = gptr(v < 8 ? F[v] : last)[m];
+  };
+  double src[NVMAX] = {};
+  if (GRAV) {
+    if (PARK) {
+      const Cell q = parked_cell<MAG>(park);
+      grav_source(D, m, src, &q);
+    } else {
+      grav_source(D, m, src);
+    }
+  }
+  fence();
+  double acc[NVMAX];
+  {
+    double div[3][NVMAX];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      // inactive directions contribute idxi*(0-0) = +0 (allocations.f90:214-240)
+#pragma unroll
+      for (int v = 0; v < nv; ++v) div[a][v] = LD == a ? duL[v] : 0.0;
+      if (LD != a && D.solve[a]) load(D.DU[a], div[a]);
+    }
+#pragma unroll
+    for (int v = 0; v < nv; ++v) {
+      acc[v] = ((div[0][v] + div[1][v]) + div[2][v]) + src[v];
+      asm volatile("" : "+v"(acc[v]));  // summed here, not where it is used
+    }
+  }
+  fence();
+  double u[NVMAX], u0[NVMAX], un[NVMAX];
+  double dt = gptr(D.sc)->dt;
+  if (stage > 1) {
+    load(D.U0, u0);
+  } else {
+#pragma unroll
+    for (int v = 0; v < nv; ++v) u0[v] = 0.0;
+  }
+  if (PARK) {
+    const Cell q = parked_cell<MAG>(park);
+#pragma unroll
+    for (int v = 1; v < 4; ++v) u[v] = gptr(D.U[v])[m];
+    if (MAG) u[8] = gptr(psi ? D.U[8] : D.U[7])[m];
+    u[0] = q.d;
+    u[4] = q.e;
+    if (MAG) {
+#pragma unroll
+      for (int v = 5; v < 8; ++v) u[v] = q.b[v - 5];
+    }
+  } else {
+    load(D.U, u);
+  }
+  fence();
+  asm volatile("" : "+v"(dt));  // nothing waits for it before the other loads are out
+  const double ft = fact * dt;
 #pragma unroll
   for (int v = 0; v < NVMAX; ++v) {
     un[v] = 0.0;
     if (v >= nv) continue;
-    // inactive directions contribute idxi*(0-0) = +0 (allocations.f90:214-240)
-    const double a = LD == 0 ? duL[v] : (D.solve[0] ? gptr(D.DU[0][v])[m] : 0.0);
-    const double b = LD == 1 ? duL[v] : (D.solve[1] ? gptr(D.DU[1][v])[m] : 0.0);
-    const double c = LD == 2 ? duL[v] : (D.solve[2] ? gptr(D.DU[2][v])[m] : 0.0);
-    const double acc = ((a + b) + c) + (GRAV ? src[v] : 0.0);  // + src
-    double u;
-    if (qc && v == 0) u = qc->d;
-    else if (qc && v == 4) u = qc->e;
-    else if (qc && MAG && v >= 5 && v <= 7) u = qc->b[v - 5];
-    else u = gptr(D.U[v])[m];
-    double u0;
-    if (stage == 1) {
-      u0 = u;
-      // (no U0: the fused form's three state sets keep the step's starting
-      // values in their own set)
-      if (D.U0[v]) gptr(D.U0[v])[m] = u;
-    } else {
-      u0 = gptr(D.U0[v])[m];
-    }
-    un[v] = faco * u0 + facn * u + ft * acc;
-    gptr(Uo[v])[m] = un[v];
-    if (v == 0) dold = u;
+    if (stage == 1) u0[v] = u[v];
+    un[v] = faco * u0[v] + facn * u[v] + ft * acc[v];
   }
+#pragma unroll
+  for (int v = 0; v < nv; ++v) {
+    if (v == 8 && !psi) break;
+    // (no U0: the fused form's three state sets keep the step's starting
+    // values in their own set)
+    if (stage == 1 && D.U0[v]) gptr(D.U0[v])[m] = u0[v];
+    gptr(Uo[v])[m] = un[v];
+  }
+  const double dold = u[0];  // stage-start density (primitive d = u(icnt))
   // species (rungekutta.f90:61-85): spcorg = spc*uorg(icnt) at stage 1;
   // spc = (faco*spcorg + facn*spc*d + fact*dt*(divergences)) / u(icnt)
   const long N = D.ncell;
 #pragma unroll
   for (int q = 0; q < HG_SPN_MAX; ++q) {
     if (q >= D.nspc) break;
-    const double x = D.SPC[q * N + m];
-    double x0;
+    const double x = gptr(D.SPC)[q * N + m];
+    double x0 = stage > 1 ? gptr(D.SPC0)[q * N + m] : 0.0;
+    const double a = D.solve[0] ? gptr(D.DUS)[(0L * D.nspc + q) * N + m] : 0.0;
+    const double b = D.solve[1] ? gptr(D.DUS)[(1L * D.nspc + q) * N + m] : 0.0;
+    const double cz = D.solve[2] ? gptr(D.DUS)[(2L * D.nspc + q) * N + m] : 0.0;
     if (stage == 1) {
       x0 = x * dold;
-      D.SPC0[q * N + m] = x0;
-    } else {
-      x0 = D.SPC0[q * N + m];
+      gptr(D.SPC0)[q * N + m] = x0;
     }
-    const double a = D.solve[0] ? D.DUS[(0L * D.nspc + q) * N + m] : 0.0;
-    const double b = D.solve[1] ? D.DUS[(1L * D.nspc + q) * N + m] : 0.0;
-    const double cz = D.solve[2] ? D.DUS[(2L * D.nspc + q) * N + m] : 0.0;
-    D.SPC[q * N + m] = (faco * x0 + facn * x * dold + ft * ((a + b) + cz)) / un[0];
+    gptr(D.SPC)[q * N + m] = (faco * x0 + facn * x * dold + ft * ((a + b) + cz)) / un[0];
   }
   // primitive (rungekutta.f90:193-232) + internalenergy (eos.f90:805-842)
   const double d = un[0];
@@ -1473,7 +1516,7 @@ __device__ __forceinline__ void rk_cell_rt(const Dev &D, long m, int stage, doub
     b1 = un[5];
     b2 = un[6];
     b3 = un[7];
-    if (D.i9wv >= 0) gptr(Wo[WPHI])[m] = DAMP ? un[8] * damp : un[8];
+    if (psi) gptr(Wo[WPHI])[m] = DAMP ? un[8] * damp : un[8];
   }
   const double eint = get_eint(MAG, e, d, v1, v2, v3, b1, b2, b3);
   gptr(Wo[WEINT])[m] = eint;
@@ -1518,9 +1561,8 @@ __device__ __forceinline__ void fused_rk(const Dev &D, const Axis &A, long base,
   const int nv = MAG ? (D.i9wv >= 0 ? 9 : 8) : 5;
   if (!TILE) {  // the lane's own cell, its primitives parked in LDS
     if (lane >= 2 && lane <= 61 && c >= 0 && c < n) {
-      const Cell qc = parked_cell<MAG>(lds);
-      rk_cell_rt<MAG, DIR>(D, base + (long)c * A.stride, stage, rk.faco, rk.fact, rk.facn,
-                           rk.damp, rk.cfl, rk.dampf, rk.grav, dti, cfm, du, &qc);
+      rk_cell_rt<MAG, DIR, true>(D, base + (long)c * A.stride, stage, rk.faco, rk.fact, rk.facn,
+                           rk.damp, rk.cfl, rk.dampf, rk.grav, dti, cfm, du, lds);
     }
     return;
   }
