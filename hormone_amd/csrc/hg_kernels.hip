@@ -43,6 +43,24 @@ __device__ __forceinline__ T *gptr(T *p) {
   return (T *)(__attribute__((address_space(1))) T *)p;
 }
 
+// One scalar load per 64 bytes of the launch's arguments (T leads them), all in
+// flight together.  Each launch has its own argument memory, cold to every
+// cache; the few bytes a kernel wants at a time came one memory round trip
+// after the other (Sod 500: 25.1 -> 20.2 us per step of
+// four launches; 1D MHD 1001: 37.2 -> 32.3; 128^2: 49.8 -> 46.6).  Only a
+// launch's first blocks find the scalar caches cold.
+template <class T>
+__device__ __forceinline__ void warm_args() {
+  if (blockIdx.x >= 1024) return;
+  typedef const __attribute__((address_space(4))) unsigned CWord;
+  CWord *p = (CWord *)__builtin_amdgcn_kernarg_segment_ptr();
+  unsigned x[(sizeof(T) + 63) / 64];
+#pragma unroll
+  for (unsigned q = 0; q < sizeof(x) / 4; ++q) x[q] = p[16 * q];
+#pragma unroll
+  for (unsigned q = 0; q < sizeof(x) / 4; ++q) asm volatile("" ::"s"(x[q]));
+}
+
 // The wavefront's index within its block, visibly uniform: index arithmetic
 // on it (the packed-line divisions) then runs on the scalar unit.
 __device__ __forceinline__ int wave_in_block() {
@@ -945,6 +963,7 @@ __device__ __forceinline__ void sweep_line(const Dev &D, long wave, int lane, in
 // cache.
 template <bool MAG, int LIM, bool TILE, bool SPC = false, bool EXT = false>
 __global__ __launch_bounds__(1024) void k_sweep(Dev D, int stage) {
+  warm_args<Dev>();
   extern __shared__ double lds[];
   if (gptr(D.sc)->stop) return;
   const int lane = threadIdx.x & 63;
@@ -1160,6 +1179,7 @@ __device__ __forceinline__ void sweep_line_mix(const Dev &D, long wave, int lane
 
 template <bool MAG, int LIM, bool TILE, bool SPC = false, bool EXT = false>
 __global__ __launch_bounds__(1024) void k_sweep_mix(Dev D, int stage) {
+  warm_args<Dev>();
   extern __shared__ double lds[];
   if (gptr(D.sc)->stop) return;
   const int lane = threadIdx.x & 63;
@@ -1278,6 +1298,7 @@ __device__ __forceinline__ void species_line(const Dev &D, long wave, int lane) 
 
 template <int LIM>
 __global__ __launch_bounds__(256) void k_species(Dev D) {
+  warm_args<Dev>();
   if (gptr(D.sc)->stop) return;
   const int lane = threadIdx.x & 63;
   const long wave = (long)blockIdx.x * (blockDim.x >> 6) + wave_in_block();
@@ -1538,6 +1559,7 @@ __device__ __forceinline__ void rk_cell(const Dev &D, long m, int stage, double 
 template <bool MAG, bool CFL, bool DAMP, bool GRAV>
 __global__ __launch_bounds__(256) void k_rk(Dev D, int stage, double faco, double fact,
                                             double facn, double damp) {
+  warm_args<Dev>();
   if (gptr(D.sc)->stop) return;
   const long m = (long)blockIdx.x * blockDim.x + threadIdx.x;
   double dti = __builtin_inf(), cfm = 0.0;
@@ -1596,6 +1618,7 @@ __device__ __forceinline__ void fused_rk(const Dev &D, const Axis &A, long base,
 // stage) one per block.  TH as k_sweep_dir.
 template <int DIR, bool MAG, int LIM, bool TILE, bool MIX, int TH>
 __global__ __launch_bounds__(TH, TH == SMALL_BLOCK ? 5 : 4) void k_sweep_rk(Dev D, int stage, RKArgs rk) {
+  warm_args<Dev>();
   extern __shared__ double lds[];
   if (gptr(D.sc)->stop) return;
   const int lane = threadIdx.x & 63;
@@ -1848,23 +1871,37 @@ __global__ __launch_bounds__(256) void k_cfl(Dev D) {
 // clipped to t_out / t_end as the reference does; ch = max fast speed.
 // One block of up to 1024 threads; each thread folds every blockDim-th
 // partial pair, four loads in flight.
-__device__ __forceinline__ void cfl_final(const Dev &D) {
-  Scalars *sc = D.sc;
-  if (sc->stop) return;
+// the scalars that end a step, read together
+struct Clock {
+  double time, t_out, t_end, dt_out, dt;
+  long long tn, tnlim, tn_out, steps_left;
+  unsigned long long err;
+  int outstyle, endstyle, stop;
+};
+__device__ __forceinline__ Clock read_clock(const Scalars *p) {
+  const auto sc = gptr(p);
+  return {sc->time, sc->t_out,  sc->t_end,      sc->dt_out, sc->dt,       sc->tn,      sc->tnlim,
+          sc->tn_out, sc->steps_left, sc->err, sc->outstyle, sc->endstyle, sc->stop};
+}
+
+// minimum and maximum over the CFL partials, to thread 0
+__device__ __forceinline__ void cfl_reduce(const Dev &D, double &a, double &b) {
   __shared__ double smin[16], smax[16];
-  double a = __builtin_inf(), b = 0.0;
-  const double2 *P = reinterpret_cast<const double2 *>(D.part);
+  a = __builtin_inf();
+  b = 0.0;
+  const auto P = gptr(reinterpret_cast<const double2 *>(D.part));
   const int nb = D.nblk_cfl, st = blockDim.x;
+  auto take = [&](double2 p) {
+    a = mn2(a, p.x);
+    b = mx2(b, p.y);
+  };
   int q = threadIdx.x;
   for (; q + 3 * st < nb; q += 4 * st) {
-    const double2 p0 = P[q], p1 = P[q + st], p2 = P[q + 2 * st], p3 = P[q + 3 * st];
-    a = mn2(mn2(mn2(mn2(a, p0.x), p1.x), p2.x), p3.x);
-    b = mx2(mx2(mx2(mx2(b, p0.y), p1.y), p2.y), p3.y);
+    const double2 p0{P[q].x, P[q].y}, p1{P[q + st].x, P[q + st].y};
+    const double2 p2{P[q + 2 * st].x, P[q + 2 * st].y}, p3{P[q + 3 * st].x, P[q + 3 * st].y};
+    take(p0), take(p1), take(p2), take(p3);
   }
-  for (; q < nb; q += st) {
-    a = mn2(a, P[q].x);
-    b = mx2(b, P[q].y);
-  }
+  for (; q < nb; q += st) take(double2{P[q].x, P[q].y});
   a = wave_min(a);
   b = wave_max(b);
   const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -1880,63 +1917,65 @@ __device__ __forceinline__ void cfl_final(const Dev &D) {
       a = mn2(a, smin[q]);
       b = mx2(b, smax[q]);
     }
-    sc->dtimin = a;
-    sc->cfmax = b;
-    double dt = D.courant * a;
-    const double time = sc->time, t_out = sc->t_out, t_end = sc->t_end;
-    if (sc->outstyle == 1) {
-      double t_ref = t_out;  // left unset by the reference unless endstyle == 1
-      if (sc->endstyle == 1) t_ref = mn2(t_out, t_end);
-      if (t_ref - time - dt > 0.0 && t_ref - time - 2.0 * dt < 0.0)
-        dt = 0.5 * (t_ref - time);
-      else
-        dt = mn2(dt, t_out - time);
-    }
-    if (sc->endstyle == 1) dt = mn2(dt, t_end - time);
-    sc->dt = dt;
-    sc->ch = b;
-    sc->chr = fden(b).r;
   }
 }
 
+// the step's dt and ch from the reduction (one thread)
+__device__ __forceinline__ void cfl_set(const Dev &D, const Clock &t, double a, double b) {
+  const auto sc = gptr(D.sc);
+  sc->dtimin = a;
+  sc->cfmax = b;
+  double dt = D.courant * a;
+  if (t.outstyle == 1) {
+    double t_ref = t.t_out;  // left unset by the reference unless endstyle == 1
+    if (t.endstyle == 1) t_ref = mn2(t.t_out, t.t_end);
+    if (t_ref - t.time - dt > 0.0 && t_ref - t.time - 2.0 * dt < 0.0)
+      dt = 0.5 * (t_ref - t.time);
+    else
+      dt = mn2(dt, t.t_out - t.time);
+  }
+  if (t.endstyle == 1) dt = mn2(dt, t.t_end - t.time);
+  sc->dt = dt;
+  sc->ch = b;
+  sc->chr = fden(b).r;
+}
+
+__device__ __forceinline__ void cfl_final(const Dev &D) {
+  const Clock t = read_clock(D.sc);
+  if (t.stop) return;
+  double a, b;
+  cfl_reduce(D, a, b);
+  if (threadIdx.x == 0) cfl_set(D, t, a, b);
+}
 __global__ __launch_bounds__(1024) void k_cfl_final(Dev D) { cfl_final(D); }
 
 // End of one main-loop iteration (hormone.f90:147-177): advance the clock,
 // then the end and output checks in the reference's order.
-__device__ __forceinline__ void step_end(const Dev &D) {
-  Scalars *sc = D.sc;
-  if (sc->stop) return;
-  if (sc->err != NOERR) {
-    sc->stop = STOP_ERROR;
+// t.stop: whether and why the run stops here
+__device__ __forceinline__ void step_end(const Dev &D, Clock &t) {
+  const auto sc = gptr(D.sc);
+  if (t.err != NOERR) {
+    sc->stop = t.stop = STOP_ERROR;
     return;
   }
-  sc->time = sc->time + sc->dt;
-  sc->tn = sc->tn + 1;
-  sc->steps_left = sc->steps_left - 1;
-  if (sc->endstyle == 1) {
-    if (sc->time >= sc->t_end) {
-      sc->stop = STOP_END;
-      return;
-    }
-  } else if (sc->endstyle == 2) {
-    if (sc->tn >= sc->tnlim) {
-      sc->stop = STOP_END;
-      return;
-    }
+  t.time = t.time + t.dt;
+  t.tn = t.tn + 1;
+  t.steps_left = t.steps_left - 1;
+  if ((t.endstyle == 1 && t.time >= t.t_end) || (t.endstyle == 2 && t.tn >= t.tnlim)) {
+    t.stop = STOP_END;
+  } else if (t.outstyle == 1 && t.time >= t.t_out) {
+    t.t_out = t.t_out + t.dt_out;
+    t.stop = STOP_OUTPUT;
+  } else if (t.outstyle == 2 && t.tn != 0 && t.tn % t.tn_out == 0) {
+    t.stop = STOP_OUTPUT;
+  } else if (t.steps_left <= 0) {
+    t.stop = STOP_MAXSTEPS;
   }
-  if (sc->outstyle == 1) {
-    if (sc->time >= sc->t_out) {
-      sc->t_out = sc->t_out + sc->dt_out;
-      sc->stop = STOP_OUTPUT;
-      return;
-    }
-  } else if (sc->outstyle == 2) {
-    if (sc->tn != 0 && sc->tn % sc->tn_out == 0) {
-      sc->stop = STOP_OUTPUT;
-      return;
-    }
-  }
-  if (sc->steps_left <= 0) sc->stop = STOP_MAXSTEPS;
+  sc->time = t.time;
+  sc->t_out = t.t_out;
+  sc->tn = t.tn;
+  sc->steps_left = t.steps_left;
+  sc->stop = t.stop;
 }
 
 
@@ -2088,11 +2127,22 @@ __global__ __launch_bounds__(256) void k_brk(Batch B, int stage, double faco, do
 }
 
 // The end of one step and the dt of the next in one launch: step_end on one
-// thread, then (if the run goes on) the CFL reduction of cfl_final.
+// thread, then (if the run goes on) cfl_set.  The clock and the partials are
+// read together.  False if the run had stopped before this step.
+__device__ __forceinline__ bool step_end_cfl(const Dev &D) {
+  Clock t = read_clock(D.sc);
+  if (t.stop) return false;
+  double a, b;
+  cfl_reduce(D, a, b);
+  if (threadIdx.x == 0) {
+    step_end(D, t);
+    if (!t.stop) cfl_set(D, t, a, b);
+  }
+  return true;
+}
 __global__ __launch_bounds__(1024) void k_step_end_cfl(Dev D) {
-  if (threadIdx.x == 0) step_end(D);
-  __syncthreads();
-  cfl_final(D);
+  warm_args<Dev>();
+  step_end_cfl(D);
 }
 
 // One block per box: close its step, then compute its next dt and ch.  In
@@ -2100,15 +2150,10 @@ __global__ __launch_bounds__(1024) void k_step_end_cfl(Dev D) {
 // start) now holds its state in the set its last stage wrote.
 __global__ __launch_bounds__(256) void k_bstep_end_cfl(Batch B) {
   const int q = blockIdx.x;
-  const Dev &D = B.boxes[B.fused ? 9 * q : q];
-  if (threadIdx.x == 0) {
-    const bool ran = gptr(D.sc)->stop == STOP_NONE;
-    step_end(D);
-    // the last stage wrote set p+1 (one or three stages) or p+2 (two)
-    if (B.fused && ran) B.bpar[q] = (B.bpar[q] + (B.rk == 2 ? 2 : 1)) % 3;
-  }
-  __syncthreads();
-  cfl_final(D);
+  typedef const __attribute__((address_space(4))) Dev CDev;
+  const bool ran = step_end_cfl(*(const Dev *)((CDev *)B.boxes + (B.fused ? 9 * q : q)));
+  // the last stage wrote set p+1 (one or three stages) or p+2 (two)
+  if (threadIdx.x == 0 && B.fused && ran) B.bpar[q] = (B.bpar[q] + (B.rk == 2 ? 2 : 1)) % 3;
 }
 
 // The slopes' grid factors of one axis, evaluated once per context from the
