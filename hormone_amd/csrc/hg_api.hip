@@ -906,6 +906,29 @@ extern "C" int hg_gravity(hg_ctx *c, double time, double dt, double *grvtime, do
   return HG_OK;
 }
 
+// What a stage of a fused step reads and writes (Dev::cons, Dev::mid).  The
+// x-fused sweep is bound by memory bandwidth, and v, e_int and W's psi of the
+// states between the stages are 5 of the 14 fields it writes and 4 of the 40 it
+// reads.  Without them, with v and e_int computed by the sweeps that read the
+// state: fused sweep of 256^3 1,409 -> 1,246 us, y and z sweeps 1,684 -> 1,685,
+// 9,345 -> 8,850 us per step; 160^3 hydro 929 -> 875, 97x131x75 568 -> 538.
+// Boxes of up to 2^19 cells stay in the Infinity Cache and would only lose
+// (512^2 121.6 -> 123.8).  All fields are kept as well in boxes whose scalar and
+// vector boundary codes take a ghost from different cells, by the sweeps fused
+// along y or z, by FP32-mixed and in batches (1.5% for one of 1e6 cells, against
+// twice the kernels).
+static void set_stage_form(Dev &D, int stage, int rk) {
+  auto source = [](int code) { return code < 2 ? code : 2; };  // as ghost_src
+  bool one = D.fdir == 0 && !D.mixed && D.ncell > 1L << 19;
+  for (int a = 0; a < 3; ++a) {
+    const Axis &A = D.ax[a];
+    one = one && (!D.solve[a] || (source(A.sc_lo) == source(A.vc_lo) &&
+                                  source(A.sc_hi) == source(A.vc_hi)));
+  }
+  D.cons = one && stage > 1;
+  D.mid = one && stage < rk;
+}
+
 // The roles of the fused form's state sets after one step: the set the last
 // stage wrote (the second for one or three stages, the third for two) trades
 // places with the current one.  Turning twice changes nothing.
@@ -985,6 +1008,7 @@ static int enqueue_stages(hg_ctx *c, bool fuse_tail, double damp, bool sweep1_do
         Df.W[w] = in.W[w];
         Df.Wo[w] = out.W[w];
       }
+      set_stage_form(Df, stage, rk);
       const int g = launch_fused_stage(Df, stage, a, c->stream, e0, e1, pre ? 2 : 0);
       if (last && fuse_tail) npart = g;
       continue;

@@ -67,12 +67,27 @@ __device__ __forceinline__ int wave_in_block() {
   return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 }
 
-// The lane's index, computed where it is asked for: a value kept from the start
-// of a sweep takes a register the solver needs.
+// The lane's and the thread's index, computed where they are asked for: values
+// kept from the start of a sweep take registers the solver needs.  TILE: from
+// threadIdx.x, whose register the tile's addresses need anyway; the lane path
+// computes the lane, so that threadIdx.x is not kept either (it was spilled and
+// loaded back eight times in the fused x sweep).
+template <bool TILE>
 __device__ __forceinline__ int lane_again() {
-  int t = threadIdx.x;
-  asm volatile("" : "+v"(t));
-  return t & 63;
+  if (TILE) {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t & 63;
+  }
+  unsigned all = ~0u;
+  asm volatile("" : "+s"(all));
+  return (int)__builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0u));
+}
+// wave_in_block() for use after the solver, in a scalar register
+__device__ __forceinline__ int wave_kept() {
+  int w = wave_in_block();
+  asm volatile("" : "+s"(w));
+  return w;
 }
 
 struct Cell {
@@ -126,13 +141,39 @@ __device__ __forceinline__ Cell finish_cell(const Dev &D, const Axis &A, int c,
     q.eint = f[WEINT];
     q.e = f[WE];
   } else {
-    const double gm1 = D.gamma - 1.0;
+    const double gm1 = gam_1(D.gamma);
     const double p = sc >= 4 ? f[WEINT] : gm1 * f[WEINT];
     q.eint = p / gm1;
     q.e = q.eint + 0.5 * (q.d * (q.v[0] * q.v[0] + q.v[1] * q.v[1] + q.v[2] * q.v[2]) +
                           q.b[0] * q.b[0] + q.b[1] * q.b[1] + q.b[2] * q.b[2]);
   }
   return q;
+}
+
+// The conserved state D.U holds between the stages of a fused step (Dev::cons):
+// from d, m, e and B of a cell to its velocities and internal energy, as the RK
+// update computes them (rk_cell_rt).  FAST: without operand scaling; the
+// sweep's own tests cover it (Chk).
+template <bool MAG, bool FAST>
+__device__ __forceinline__ void cons_prims(double f[NWMAX]) {
+  if (FAST) {
+    const Den64 d = fden(f[WD]);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) f[WV1 + a] = fdiv_(d, f[WV1 + a]);
+  } else {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) f[WV1 + a] = f[WV1 + a] / f[WD];
+  }
+  f[WEINT] = get_eint(MAG, f[WE], f[WD], f[WV1], f[WV2], f[WV3], MAG ? f[WB1] : 0.0,
+                      MAG ? f[WB2] : 0.0, MAG ? f[WB3] : 0.0);
+}
+
+// where field w of the state is: momenta for velocities and U's psi if CONS
+template <bool CONS>
+__device__ __forceinline__ const double *state_field(const Dev &D, int w) {
+  if (w >= WV1 && w <= WV3) return CONS ? D.U[1 + (w - WV1)] : D.W[w];
+  if (w == WPHI) return CONS && D.i9wv >= 0 ? D.U[8] : D.W[w];
+  return D.W[w];
 }
 
 // Source rows of cell c of a line (both the cell itself when interior).
@@ -249,7 +290,7 @@ __device__ __forceinline__ void raw_cell(const Dev &D, const Axis &A, long base,
 
 // One cell read straight from HBM by its own lane.
 // EXT = false: the caller's boxes have no code 4, 5, 9 or 10 (batches).
-template <int DIR, bool MAG, bool EXT = true>
+template <int DIR, bool MAG, bool EXT, bool CONS, bool FAST>
 __device__ __forceinline__ Cell load_cell(const Dev &D, const Axis &A, long base, long line,
                                           int c) {
   if (EXT && A.ext) {
@@ -262,14 +303,15 @@ __device__ __forceinline__ Cell load_cell(const Dev &D, const Axis &A, long base
   double f[NWMAX];
   f[WD] = gptr(D.W[WD])[ms];
   f[WE] = gptr(D.W[WE])[ms];
-  f[WEINT] = gptr(D.W[WEINT])[ms];
 #pragma unroll
-  for (int a = 0; a < 3; ++a) f[WV1 + a] = gptr(D.W[WV1 + a])[mv];
+  for (int a = 0; a < 3; ++a) f[WV1 + a] = gptr(state_field<CONS>(D, WV1 + a))[mv];
   if (MAG) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) f[WB1 + a] = gptr(D.W[WB1 + a])[mv];
-    f[WPHI] = gptr(D.W[WPHI])[ms];
+    f[WPHI] = gptr(state_field<CONS>(D, WPHI))[ms];
   }
+  if (CONS) cons_prims<MAG, FAST>(f);
+  else f[WEINT] = gptr(D.W[WEINT])[ms];
   return finish_cell<DIR, MAG>(D, A, c, f);
 }
 
@@ -310,11 +352,12 @@ __device__ __forceinline__ uint2 *tile_dst(double *lds, int nf, int bw) {
 // U[5..7] (the same buffers) and d, v feed the gravity source, so the
 // update reads none of them from memory again, and they hold no registers
 // across the flux computation.  Layout [field][thread], fields d e v1 v2
-// v3 (b1 b2 b3); each thread reads back only what it wrote.
+// v3 (b1 b2 b3); each thread reads back only what it wrote.  lds: the wavefront's
+// own 64 entries.
 __host__ __device__ inline int park_fields(bool mag) { return mag ? 8 : 5; }
 template <bool MAG>
 __device__ __forceinline__ void park_cell(double *lds, const Cell &q) {
-  double *p = lds + threadIdx.x;
+  double *p = lds + lane_again<false>();  // (addresses not kept for a second time)
   const int bs = blockDim.x;
   p[0] = q.d;
   p[bs] = q.e;
@@ -327,9 +370,7 @@ __device__ __forceinline__ void park_cell(double *lds, const Cell &q) {
 }
 template <bool MAG>
 __device__ __forceinline__ Cell parked_cell(const double *lds) {
-  int t = threadIdx.x;
-  asm volatile("" : "+v"(t));  // the addresses again, not kept from park_cell
-  const double *p = lds + t;
+  const double *p = lds + lane_again<false>();  // (again, not kept from park_cell)
   const int bs = blockDim.x;
   Cell q;
   q.d = p[0];
@@ -452,20 +493,22 @@ __device__ __forceinline__ void cell_ijk(const Dev &D, long m, int &i, int &j, i
 }
 
 // the lane's own cell of a loaded tile
-template <int DIR, bool MAG>
+template <int DIR, bool MAG, bool CONS, bool FAST>
 __device__ __forceinline__ Cell tile_column(const Dev &D, const Axis &A, int c,
                                             const double *lds) {
-  const int bw = blockDim.x >> 6, w = wave_in_block(), lane = lane_again();
+  const int bw = blockDim.x >> 6, w = wave_in_block(), lane = lane_again<true>();
   const int ld = tile_ld(bw), fs = 64 * ld;
   const int nf = MAG ? NWMAX : WEINT + 1;
   double f[NWMAX];
   const double *p = lds + lane * ld + w;
 #pragma unroll
-  for (int k = 0; k < NWMAX; ++k) f[k] = k < nf ? p[k * fs] : 0.0;
+  for (int k = 0; k < NWMAX; ++k) f[k] = k < nf && k != WEINT ? p[k * fs] : 0.0;
+  if (CONS) cons_prims<MAG, FAST>(f);
+  else f[WEINT] = p[WEINT * fs];
   return finish_cell<DIR, MAG>(D, A, c, f);
 }
 
-template <int DIR, bool MAG, bool EXT = true>
+template <int DIR, bool MAG, bool EXT, bool CONS, bool FAST>
 __device__ __forceinline__ Cell tile_cell(const Dev &D, const Axis &A, long wave0, long base,
                                           int c, bool valid, double *lds) {
   const int bw = blockDim.x >> 6, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -503,18 +546,18 @@ __device__ __forceinline__ Cell tile_cell(const Dev &D, const Axis &A, long wave
       const long ms = sv.x, mv = sv.y;
       p[WD * fs] = gptr(D.W[WD])[ms];
       p[WE * fs] = gptr(D.W[WE])[ms];
-      p[WEINT * fs] = gptr(D.W[WEINT])[ms];
+          if (!CONS) p[WEINT * fs] = gptr(D.W[WEINT])[ms];
 #pragma unroll
-      for (int a = 0; a < 3; ++a) p[(WV1 + a) * fs] = gptr(D.W[WV1 + a])[mv];
+      for (int a = 0; a < 3; ++a) p[(WV1 + a) * fs] = gptr(state_field<CONS>(D, WV1 + a))[mv];
       if (MAG) {
 #pragma unroll
         for (int a = 0; a < 3; ++a) p[(WB1 + a) * fs] = gptr(D.W[WB1 + a])[mv];
-        p[WPHI * fs] = gptr(D.W[WPHI])[ms];
+        p[WPHI * fs] = gptr(state_field<CONS>(D, WPHI))[ms];
       }
     }
   }
   __syncthreads();
-  return tile_column<DIR, MAG>(D, A, c, lds);
+  return tile_column<DIR, MAG, CONS, FAST>(D, A, c, lds);
 }
 
 // Thread t's row of the tile on the way out: true with its element index m
@@ -867,7 +910,7 @@ __device__ __forceinline__ void fused_rk(const Dev &D, const Axis &A, long base,
                                          double &cfm);
 
 template <int DIR, bool MAG, int LIM, bool TILE = false, bool SPC = false, bool FUSED = false,
-          bool EXT = true>
+          bool EXT = true, bool CONS = false>
 __device__ __forceinline__ void sweep_line(const Dev &D, long wave, int lane, int stage,
                                            double *lds = nullptr, const RKArgs *rk = nullptr,
                                            double *dti = nullptr, double *cfm = nullptr) {
@@ -882,9 +925,12 @@ __device__ __forceinline__ void sweep_line(const Dev &D, long wave, int lane, in
   long line, base;
   int c;
   lane_cell<DIR>(D, A, wave, lane, line, base, c);
-  const Cell q = TILE ? tile_cell<DIR, MAG, EXT>(D, A, wave0, base, c, valid, lds)
-                      : load_cell<DIR, MAG, EXT>(D, A, base, line, c);
-  if (FUSED && !TILE) park_cell<MAG>(lds, q);
+  const Cell q = TILE ? tile_cell<DIR, MAG, EXT, CONS, true>(D, A, wave0, base, c, valid, lds)
+                      : load_cell<DIR, MAG, EXT, CONS, true>(D, A, base, line, c);
+  if (FUSED && !TILE) {
+    lds += 64 * wave_kept();
+    park_cell<MAG>(lds, q);
+  }
   // (element indices fit in 32 bits)
   const unsigned ubase = (unsigned)base;
   const double gam = D.gamma;
@@ -894,22 +940,23 @@ __device__ __forceinline__ void sweep_line(const Dev &D, long wave, int lane, in
   const bool odd = line_faces<DIR, MAG, LIM>(A, q, c, lane, gam, Dch, t);
   // the rare branches place the lane again, so that nothing is kept for them
   auto again = [&](long &line2, long &base2, int &c2) {
-    lane_cell<DIR>(D, A, wave, lane_again(), line2, base2, c2);
+    lane_cell<DIR>(D, A, wave, lane_again<TILE>(), line2, base2, c2);
   };
   if (odd) {  // the whole wavefront: its cells again, in plain divisions
     long line2, base2;
     int c2;
     again(line2, base2, c2);
     Cell q2;
-    if (TILE) q2 = tile_column<DIR, MAG>(D, A, c2, lds);
-    else q2 = load_cell<DIR, MAG, EXT>(D, A, base2, line2, c2);
+    if (TILE) q2 = tile_column<DIR, MAG, CONS, false>(D, A, c2, lds);
+    else q2 = load_cell<DIR, MAG, EXT, CONS, false>(D, A, base2, line2, c2);
+    if (CONS && FUSED && !TILE) park_cell<MAG>(lds, q2);
     double fe[4];
     line_faces_plain<DIR, MAG, LIM>(A, q2, c2, gam, gptr(D.sc)->ch, t, fe);
     neg = fe[1] <= 0.0 || fe[0] <= 0.0 || fe[3] <= 0.0 || fe[2] <= 0.0;
   }
   const bool fxb = EXT && A.ext && flux_face(A, c);
   if (fxb) boundary_flux<DIR>(A, c, t);
-  lane = lane_again();
+  lane = lane_again<TILE>();
   // faces between lanes l and l+1 have valid slopes on both sides for l = 1..61
   const bool face_valid = valid && (c >= -1 && c <= n - 1) && lane >= 1 && lane <= 61 && !fxb;
   if (face_valid && neg) {
@@ -1036,9 +1083,12 @@ __device__ __forceinline__ void sweep_line_mix(const Dev &D, long wave, int lane
   long line, base;
   int c;
   lane_cell<DIR>(D, A, wave, lane, line, base, c);
-  const Cell q = TILE ? tile_cell<DIR, MAG, EXT>(D, A, wave0, base, c, valid, lds)
-                      : load_cell<DIR, MAG, EXT>(D, A, base, line, c);
-  if (FUSED && !TILE) park_cell<MAG>(lds, q);
+  const Cell q = TILE ? tile_cell<DIR, MAG, EXT, false, false>(D, A, wave0, base, c, valid, lds)
+                      : load_cell<DIR, MAG, EXT, false, false>(D, A, base, line, c);
+  if (FUSED && !TILE) {
+    lds += 64 * wave_kept();
+    park_cell<MAG>(lds, q);
+  }
   const double m0 = q.d * q.v[0], m1 = q.d * q.v[1], m2 = q.d * q.v[2];
   const double qd[8] = {q.d, q.e, m0, m1, m2, q.b[0], q.b[1], q.b[2]};
   const int cc = c < -2 ? -2 : (c > n + 1 ? n + 1 : c);
@@ -1222,7 +1272,7 @@ __global__ __launch_bounds__(1024) void k_sweep_mix(Dev D, int stage) {
 // would spill in every one of them (128^2: 11.3 -> 13.5 us).
 constexpr int SMALL_BLOCK = 256, LARGE_BLOCK = 1024;
 
-template <int DIR, bool MAG, int LIM, bool TILE, bool MIX, int TH>
+template <int DIR, bool MAG, int LIM, bool TILE, bool MIX, int TH, bool CONS>
 __global__ __launch_bounds__(TH, TH == SMALL_BLOCK ? 5 : 4) void k_sweep_dir(Dev D, int stage) {
   extern __shared__ double lds[];
   if (gptr(D.sc)->stop) return;
@@ -1232,7 +1282,7 @@ __global__ __launch_bounds__(TH, TH == SMALL_BLOCK ? 5 : 4) void k_sweep_dir(Dev
   // tiled: a partly filled last block runs its padding wavefronts too
   if (TILE ? w - (threadIdx.x >> 6) >= D.waves[DIR] : w >= D.waves[DIR]) return;
   if (MIX) sweep_line_mix<DIR, MAG, LIM, TILE, false, false>(D, w, lane, stage, lds);
-  else sweep_line<DIR, MAG, LIM, TILE, false, false, false>(D, w, lane, stage, lds);
+  else sweep_line<DIR, MAG, LIM, TILE, false, false, false, CONS>(D, w, lane, stage, lds);
 }
 
 // ---- advected species (compswitch 2) -----------------------------------------
@@ -1319,7 +1369,7 @@ __device__ __forceinline__ void cfl_cell(const Dev &D, long m, double d, double 
   int i, j, k;
   cell_ijk(D, m, i, j, k);
   const double gam = D.gamma;
-  const double p = (gam - 1.0) * eint;
+  const double p = gam_1(gam) * eint;
   const double cs = sqrt(gam * p / d);
   double cf1, cf2, cf3;
   if (MAG) {
@@ -1354,17 +1404,17 @@ __device__ __forceinline__ double wave_max(double x) {
 
 // block (up to 1024 threads) reduction of (min dti, max cf) into D.part[blk]
 __device__ __forceinline__ void cfl_block_reduce(const Dev &D, double dti, double cfm,
-                                                 long blk) {
+                                                 long blk, int w = wave_in_block()) {
   __shared__ double smin[16], smax[16];
   dti = wave_min(dti);
   cfm = wave_max(cfm);
-  const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
+  const int lane = lane_again<false>(), nw = blockDim.x >> 6;
+  if (lane == 0) {
     smin[w] = dti;
     smax[w] = cfm;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (w == 0 && lane == 0) {
     double a = smin[0], b = smax[0];
     for (int q = 1; q < nw; ++q) {
       a = mn2(a, smin[q]);
@@ -1529,18 +1579,21 @@ __device__ __forceinline__ void rk_cell_rt(const Dev &D, long m, int stage, doub
   const double v1 = un[1] / d, v2 = un[2] / d, v3 = un[3] / d;
   const double e = un[4];
   // W[d], W[e] and W[B] are U[0], U[4] and U[5..7] (same buffers)
-  gptr(Wo[WV1])[m] = v1;
-  gptr(Wo[WV2])[m] = v2;
-  gptr(Wo[WV3])[m] = v3;
+  const bool prim = LD < 0 || !D.mid;
+  if (prim) {
+    gptr(Wo[WV1])[m] = v1;
+    gptr(Wo[WV2])[m] = v2;
+    gptr(Wo[WV3])[m] = v3;
+  }
   double b1 = 0, b2 = 0, b3 = 0;
   if (MAG) {
     b1 = un[5];
     b2 = un[6];
     b3 = un[7];
-    if (psi) gptr(Wo[WPHI])[m] = DAMP ? un[8] * damp : un[8];
+    if (psi && prim) gptr(Wo[WPHI])[m] = DAMP ? un[8] * damp : un[8];
   }
   const double eint = get_eint(MAG, e, d, v1, v2, v3, b1, b2, b3);
-  gptr(Wo[WEINT])[m] = eint;
+  if (prim) gptr(Wo[WEINT])[m] = eint;
   if (eint <= 0.0) {
     int i, j, k;
     cell_ijk(D, m, i, j, k);
@@ -1616,23 +1669,24 @@ __device__ __forceinline__ void fused_rk(const Dev &D, const Axis &A, long base,
 
 // One wavefront per segment of a DIR line, as k_sweep; CFL partials (last
 // stage) one per block.  TH as k_sweep_dir.
-template <int DIR, bool MAG, int LIM, bool TILE, bool MIX, int TH>
+template <int DIR, bool MAG, int LIM, bool TILE, bool MIX, int TH, bool CONS>
 __global__ __launch_bounds__(TH, TH == SMALL_BLOCK ? 5 : 4) void k_sweep_rk(Dev D, int stage, RKArgs rk) {
   warm_args<Dev>();
   extern __shared__ double lds[];
   if (gptr(D.sc)->stop) return;
   const int lane = threadIdx.x & 63;
-  const long wave = (long)blockIdx.x * (blockDim.x >> 6) + wave_in_block();
+  const int w = wave_kept();
+  const long wave = (long)blockIdx.x * (blockDim.x >> 6) + w;
   double dti = __builtin_inf(), cfm = 0.0;
   if (TILE || wave < D.waves[DIR]) {
     if (MIX)
       sweep_line_mix<DIR, MAG, LIM, TILE, false, false, true>(D, wave, lane, stage, lds, &rk,
                                                                &dti, &cfm);
     else
-      sweep_line<DIR, MAG, LIM, TILE, false, true, false>(D, wave, lane, stage, lds, &rk, &dti,
+      sweep_line<DIR, MAG, LIM, TILE, false, true, false, CONS>(D, wave, lane, stage, lds, &rk, &dti,
                                                            &cfm);
   }
-  if (rk.cfl) cfl_block_reduce(D, dti, cfm, blockIdx.x);
+  if (rk.cfl) cfl_block_reduce(D, dti, cfm, blockIdx.x, w);
 }
 
 // ---- pressure(): eint from e, d, v, B after an upload ---------------------
@@ -2464,15 +2518,26 @@ static void sweep_rk_variant(const Dev &D, int stage, const RKArgs &rk, unsigned
                              size_t tile, hipStream_t s, const KEv *ev) {
   if constexpr (DIR > 0) {  // x lines are lane lines, never tiled
     if (tile) {
-      if (D.mixed) klaunch_lds(k_sweep_rk<DIR, MAG, LIM, true, true, TH>, g, bs, tile, s, ev, D, stage, rk);
-      else klaunch_lds(k_sweep_rk<DIR, MAG, LIM, true, false, TH>, g, bs, tile, s, ev, D, stage, rk);
+      if (D.mixed) klaunch_lds(k_sweep_rk<DIR, MAG, LIM, true, true, TH, false>, g, bs, tile, s, ev, D, stage, rk);
+      else klaunch_lds(k_sweep_rk<DIR, MAG, LIM, true, false, TH, false>, g, bs, tile, s, ev, D, stage, rk);
       return;
     }
   }
   // the lane path parks each thread's primitives (park_cell)
   const size_t park = (size_t)park_fields(MAG) * sizeof(double) * (size_t)bs;
-  if (D.mixed) klaunch_lds(k_sweep_rk<DIR, MAG, LIM, false, true, TH>, g, bs, park, s, ev, D, stage, rk);
-  else klaunch_lds(k_sweep_rk<DIR, MAG, LIM, false, false, TH>, g, bs, park, s, ev, D, stage, rk);
+  if constexpr (DIR == 0) {
+    if (D.cons) {
+      klaunch_lds(k_sweep_rk<DIR, MAG, LIM, false, false, TH, true>, g, bs, park, s, ev, D, stage,
+                  rk);
+      return;
+    }
+  }
+  if (D.mixed)
+    klaunch_lds(k_sweep_rk<DIR, MAG, LIM, false, true, TH, false>, g, bs, park, s, ev, D, stage,
+                rk);
+  else
+    klaunch_lds(k_sweep_rk<DIR, MAG, LIM, false, false, TH, false>, g, bs, park, s, ev, D, stage,
+                rk);
 }
 
 template <int DIR, int TH>
@@ -2501,12 +2566,15 @@ static void sweep_dir_th(const Dev &D, int stage, int bs, size_t tile, hipStream
                          const KEv *ev) {
   const unsigned g = nblk(D.waves[DIR], bs / 64);
   const bool t = DIR > 0 && tile;
-  if (D.mixed) {
-    if (t) klaunch_lds(k_sweep_dir<DIR, MAG, LIM, true, true, TH>, g, bs, tile, s, ev, D, stage);
-    else klaunch_lds(k_sweep_dir<DIR, MAG, LIM, false, true, TH>, g, bs, 0, s, ev, D, stage);
+  if (D.cons) {
+    if (t) klaunch_lds(k_sweep_dir<DIR, MAG, LIM, true, false, TH, true>, g, bs, tile, s, ev, D, stage);
+    else klaunch_lds(k_sweep_dir<DIR, MAG, LIM, false, false, TH, true>, g, bs, 0, s, ev, D, stage);
+  } else if (D.mixed) {
+    if (t) klaunch_lds(k_sweep_dir<DIR, MAG, LIM, true, true, TH, false>, g, bs, tile, s, ev, D, stage);
+    else klaunch_lds(k_sweep_dir<DIR, MAG, LIM, false, true, TH, false>, g, bs, 0, s, ev, D, stage);
   } else {
-    if (t) klaunch_lds(k_sweep_dir<DIR, MAG, LIM, true, false, TH>, g, bs, tile, s, ev, D, stage);
-    else klaunch_lds(k_sweep_dir<DIR, MAG, LIM, false, false, TH>, g, bs, 0, s, ev, D, stage);
+    if (t) klaunch_lds(k_sweep_dir<DIR, MAG, LIM, true, false, TH, false>, g, bs, tile, s, ev, D, stage);
+    else klaunch_lds(k_sweep_dir<DIR, MAG, LIM, false, false, TH, false>, g, bs, 0, s, ev, D, stage);
   }
 }
 

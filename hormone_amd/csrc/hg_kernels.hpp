@@ -104,6 +104,10 @@ struct Dev {
   // new state to the other buffer set Uo/Wo (W aliasing U as above)
   int fdir;        // the direction fused with the RK update, -1 if none
   double *Uo[NVMAX], *Wo[NWMAX];
+  // Between the stages of an x-fused step only U may be kept (set_stage_form): a
+  // stage whose input was written that way (cons) computes v and e_int from it,
+  // one that writes its output that way (mid) stores neither them nor W's psi
+  int cons, mid;
   double *part;    // CFL partials: 2 doubles per block of 256 cells
   Scalars *sc;
   int nblk_cfl;

@@ -129,6 +129,13 @@ __device__ __forceinline__ R modified_mc(R u0, R u1, R u2, R xm, R x0, R xp,
   return modified_mc_d(u0, u1, u2, xp - x0, cf, cb, mkden<false>(x0 - xm), mkden<false>(xp - x0));
 }
 
+// gamma - 1 where it is used: one value for a whole sweep was kept in a register
+// pair across the solver, and spilled
+__device__ __forceinline__ double gam_1(double gam) {
+  asm volatile("" : "+s"(gam));
+  return gam - 1.0;
+}
+
 // get_eint, eos.f90:846-865
 template <class R>
 __device__ __forceinline__ R get_eint(bool mag, R etot, R d, R v1, R v2, R v3, R b1,
@@ -645,7 +652,7 @@ __device__ __forceinline__ void face_fast(const double L[8], const double R_[8],
     o.b1 = MAG ? F[5 + a_] : 0.0;
     o.b2 = MAG ? F[5 + b_] : 0.0;
     o.b3 = MAG ? F[5 + c_] : 0.0;
-    o.pt = (gam - 1.0) * get_eint(MAG, F[1], F[0], o.v1, o.v2, o.v3, o.b1, o.b2, o.b3);
+    o.pt = gam_1(gam) * get_eint(MAG, F[1], F[0], o.v1, o.v2, o.v3, o.b1, o.b2, o.b3);
     const double as = fdiv_(Df, gam * o.pt);
     k.pos(as);
     o.cf = fsqrt(as);
