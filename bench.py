@@ -325,7 +325,7 @@ def stage_bytes(nv, rktype, grav):
     return tot / rktype + (8.0 if grav else 0.0)
 
 
-def kernel_bytes(fused, nv, nw, dim, mag, rktype=3):
+def kernel_bytes(fused, nv, nw, dim, mag, rktype=3, conserved=False):
     """Bytes per cell the stage's own launches move (their reads and writes,
     intermediates included), averaged over the stages: the sweep reads the
     primitives once per direction and writes one divergence per direction;
@@ -333,10 +333,18 @@ def kernel_bytes(fused, nv, nw, dim, mag, rktype=3):
     primitive fields that do not alias U (stage 1 writes U0 instead of
     reading it: the same count).  The fused launch reads its direction's
     primitives instead of its divergence, and with its three state sets it
-    stores no U0: stage 1 neither reads nor writes one."""
+    stores no U0: stage 1 neither reads nor writes one.  conserved: between
+    its stages the x-fused form keeps U only (FP64 boxes of more than 2^19
+    cells), so later stages read that once and only the last writes the
+    other primitive fields."""
     aliased = 5 if mag else 2
     wr = nw - aliased
-    if fused:
+    if fused and conserved:
+        mid = (rktype - 1) / rktype
+        read = nw / rktype + nv * mid
+        sweep = (dim - 1) * (read + nv) * 8
+        rk = (read + (nv - aliased) / rktype + (dim - 1) * nv + nv + nv * mid + wr / rktype) * 8
+    elif fused:
         sweep = (dim - 1) * (nw + nv) * 8
         rk = (nw + (dim - 1) * nv + 2 * nv + nv * (rktype - 1) / rktype + wr) * 8
     else:
@@ -407,7 +415,8 @@ def roofline(a, r):
                "k_sweep" + ("_mix" if prm.precision == "fp32mix" else ""))
     rk_k = "k_sweep_rk" if fused else "k_rk"
     b_alg = stage_bytes(nv, prm.rktype, grav) * g.ncells
-    sb, rb = kernel_bytes(fused, nv, nw, dim, prm.mag_on, prm.rktype)
+    sb, rb = kernel_bytes(fused, nv, nw, dim, prm.mag_on, prm.rktype,
+                          fused == 2 and prm.precision == "fp64" and g.ncells > 1 << 19)
     us = us_s + us_r
     ach = b_alg / (us * 1e-6) / 1e9
     key = f"{workload_key(a, prm)}/{prm.precision}"
