@@ -301,10 +301,10 @@ def tune(a, eng, run):
     fused = 0
     if a.sweep_waves:
         eng.set_launch(a.sweep_waves)
-    if a.fused in ("last", "x"):
-        fused = {"last": 1, "x": 2}[a.fused]
+    if a.fused in ("last", "x", "off"):  # a context starts in the form of its size
+        fused = {"last": 1, "x": 2, "off": 0}[a.fused]
         eng.set_fused(fused)
-        tuned["fused_sweep"] = a.fused
+        tuned["fused_sweep"] = names[fused]
     elif a.fused == "auto":
         fused, ftimes = tune_fused(eng, run.advance, steps=max(2, min(8, a.warmup // 4)))
         tuned["fused_sweep"] = names[fused]
