@@ -12,6 +12,8 @@
 !
 ! The switch is a namelist group of its own in the parameter file,
 !   &gpucon use_gpu=.true. fused=2 /
+! (fused: the argument of hg_set_fused, 0 separate, 1 the last direction, 2 x; a
+! negative value leaves the context in the form it starts with),
 ! read like setup.f90:154-165 reads each group (iostat, so a file without
 ! it leaves the defaults).  With use_gpu = .false. every gpu_* call is the
 ! reference's own routine, unchanged.
@@ -24,7 +26,7 @@ module gpu_bridge
           gpu_sync, use_gpu
 
  logical,save:: use_gpu = .false.
- integer,save:: fused = 0, sweep_waves = 0, mixed = 0, device = 0
+ integer,save:: fused = -1, sweep_waves = 0, mixed = 0, device = 0
  type(c_ptr),save:: hctx = c_null_ptr
 
  namelist /gpucon/ use_gpu, fused, sweep_waves, mixed, device
@@ -68,7 +70,7 @@ contains
   st = hg_create_cartesian(desc, hctx, x1, xi1, dx1, dxi1, idx1, idxi1, &
                            x2, xi2, dx2, dxi2, idx2, idxi2, x3, xi3, dx3, dxi3, idx3, idxi3)
   call hg_check(hctx, st, 'hg_create')
-  if(fused/=0)call hg_check(hctx, hg_set_fused(hctx, int(fused,c_int32_t)), 'hg_set_fused')
+  if(fused>=0)call hg_check(hctx, hg_set_fused(hctx, int(fused,c_int32_t)), 'hg_set_fused')
   if(sweep_waves/=0) &
    call hg_check(hctx, hg_set_launch(hctx, int(sweep_waves,c_int32_t)), 'hg_set_launch')
 

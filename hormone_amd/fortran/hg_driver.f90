@@ -54,7 +54,8 @@ program hg_driver
  character(len=256):: outfile='final.bin', initfile=''
  logical:: is_test=.true.
  integer:: device=0
- integer:: fused=0             ! hg_set_fused: 0 off, 1 last direction, 2 x
+ integer:: fused=-1            ! hg_set_fused: 0 off, 1 last direction, 2 x;
+                               ! negative: as the context starts
  real(8):: gconst=6.67430d-8   ! G (a parameter of the reference, G=1 for test set-ups)
 
  namelist /gridcon/ xi1s,xi1e,xi2s,xi2e,xi3s,xi3e,is,ie,js,je,ks,ke, &
@@ -174,7 +175,7 @@ program hg_driver
  st = hg_create_cartesian(desc, ctx, x1, xi1, dx1, dxi1, idx1, idxi1, &
                           x2, xi2, dx2, dxi2, idx2, idxi2, x3, xi3, dx3, dxi3, idx3, idxi3)
  call hg_check(ctx, st, 'hg_create')
- if(fused/=0)then
+ if(fused>=0)then
   st = hg_set_fused(ctx, int(fused, c_int32_t)) ; call hg_check(ctx, st, 'hg_set_fused')
  end if
  st = hg_upload(ctx, HG_F_D, d)   ; call hg_check(ctx, st, 'upload')
