@@ -735,6 +735,28 @@ extern "C" int hg_profile(hg_ctx *c, int32_t enable) {
   return HG_OK;
 }
 
+// Whether a fused step keeps only the conserved fields between its stages.  The
+// x-fused sweep is bound by memory bandwidth, and v, e_int and W's psi of the
+// states between the stages are 5 of the 14 fields it writes and 4 of the 40 it
+// reads.  Without them, with v and e_int computed by the sweeps that read the
+// state: fused sweep of 256^3 1,409 -> 1,246 us, y and z sweeps 1,684 -> 1,685,
+// 9,345 -> 8,850 us per step; 160^3 hydro 929 -> 875, 97x131x75 568 -> 538.
+// Boxes of up to 2^19 cells stay in the Infinity Cache and would only lose
+// (512^2 121.6 -> 123.8).  All fields are kept as well in boxes whose scalar and
+// vector boundary codes take a ghost from different cells, by the sweeps fused
+// along y or z, by FP32-mixed and in batches (1.5% for one of 1e6 cells, against
+// twice the kernels).
+static bool conserved_stages(const Dev &D) {
+  auto source = [](int code) { return code < 2 ? code : 2; };  // as ghost_src
+  bool one = D.fdir == 0 && !D.mixed && D.ncell > 1L << 19;
+  for (int a = 0; a < 3; ++a) {
+    const Axis &A = D.ax[a];
+    one = one && (!D.solve[a] || (source(A.sc_lo) == source(A.vc_lo) &&
+                                  source(A.sc_hi) == source(A.vc_hi)));
+  }
+  return one;
+}
+
 extern "C" int hg_profile_read(const hg_ctx *c, int32_t kind, double *ms_total,
                                int64_t *launches, double *bytes_per_launch) {
   if (!c || kind < 0 || kind >= HG_PROF_N) return HG_ERR_ARG;
@@ -746,19 +768,31 @@ extern "C" int hg_profile_read(const hg_ctx *c, int32_t kind, double *ms_total,
   // fused one
   const bool fused = fused_now(c);
   const int nsw = D.dim - (fused ? 1 : 0);
+  const int rk = c->desc.rktype;
+  // the share of the stages that read conserved fields only, and what the
+  // sweep of one direction then reads
+  const bool cons = fused && rk > 1 && conserved_stages(D);
+  const double later = cons ? (double)(rk - 1) / rk : 0.0;
+  const double read = (1.0 - later) * D.nw + later * D.nv;
   double bytes = 0.0;
   switch (kind) {
-    case HG_PROF_SWEEP:  // read the primitives once and write one divergence per direction
-      bytes = cell * (double)nsw * (D.nw + D.nv);
+    case HG_PROF_SWEEP:  // read the state once and write one divergence per direction
+      bytes = cell * nsw * (read + D.nv);
       break;
     case HG_PROF_RK: {
       // read U, U0 and the swept divergences, write U and the W fields that
       // are not U (stage 1 writes U0 and reads none: the same count); the
       // fused launch also reads its direction's primitives instead of a
       // divergence, and with its three state sets stage 1 neither reads
-      // nor writes a U0 (averaged over the stages)
-      const int rk = c->desc.rktype;
-      bytes = cell * (fused ? D.nw + nsw * D.nv + 2.0 * D.nv +
+      // nor writes a U0 (averaged over the stages).  With conserved fields
+      // only between the stages, the state it reads is U itself (stage 1: the
+      // primitives and the U fields among them that W does not hold), and the
+      // last stage alone writes the other W fields.
+      if (cons)
+        bytes = cell * (read + (D.nv - (D.nw - wr)) / (double)rk + nsw * D.nv + D.nv +
+                        later * D.nv + wr / (double)rk);
+      else
+        bytes = cell * (fused ? D.nw + nsw * D.nv + 2.0 * D.nv +
                                      (double)D.nv * (rk - 1) / rk + wr
                                : (double)(D.dim * D.nv + 3 * D.nv + wr));
       break;
@@ -906,25 +940,9 @@ extern "C" int hg_gravity(hg_ctx *c, double time, double dt, double *grvtime, do
   return HG_OK;
 }
 
-// What a stage of a fused step reads and writes (Dev::cons, Dev::mid).  The
-// x-fused sweep is bound by memory bandwidth, and v, e_int and W's psi of the
-// states between the stages are 5 of the 14 fields it writes and 4 of the 40 it
-// reads.  Without them, with v and e_int computed by the sweeps that read the
-// state: fused sweep of 256^3 1,409 -> 1,246 us, y and z sweeps 1,684 -> 1,685,
-// 9,345 -> 8,850 us per step; 160^3 hydro 929 -> 875, 97x131x75 568 -> 538.
-// Boxes of up to 2^19 cells stay in the Infinity Cache and would only lose
-// (512^2 121.6 -> 123.8).  All fields are kept as well in boxes whose scalar and
-// vector boundary codes take a ghost from different cells, by the sweeps fused
-// along y or z, by FP32-mixed and in batches (1.5% for one of 1e6 cells, against
-// twice the kernels).
+// What a stage of a fused step reads and writes (Dev::cons, Dev::mid).
 static void set_stage_form(Dev &D, int stage, int rk) {
-  auto source = [](int code) { return code < 2 ? code : 2; };  // as ghost_src
-  bool one = D.fdir == 0 && !D.mixed && D.ncell > 1L << 19;
-  for (int a = 0; a < 3; ++a) {
-    const Axis &A = D.ax[a];
-    one = one && (!D.solve[a] || (source(A.sc_lo) == source(A.vc_lo) &&
-                                  source(A.sc_hi) == source(A.vc_hi)));
-  }
+  const bool one = conserved_stages(D);
   D.cons = one && stage > 1;
   D.mid = one && stage < rk;
 }
