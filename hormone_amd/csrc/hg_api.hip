@@ -2,19 +2,18 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <vector>
 
 #include "../../include/hormone_hip.h"
 #include "hg_kernels.hpp"
+#include "hg_rows.hpp"
 
 using namespace hg;
 
@@ -571,7 +570,7 @@ static int ensure_eint(hg_ctx *c) {
 // staging memory; take(r) hands row r of it over to the caller's array.
 //
 // The copy over the bus runs at about 55 GB/s, one thread's copy out of the
-// staging memory at about 14 GB/s.  Fields of more than 2 MB are therefore
+// staging memory at about 14 GB/s.  Fields of 3 MB and more are therefore
 // staged in chunks, and threads of this call hand a chunk over while the next
 // ones arrive: 11.5 -> 3.1 ms per 256^3 field (134 MB, 43 GB/s; 3.9 ms with 4
 // threads, no better with 16), 2.7 -> 1.1 ms at 160^3, 0.66 -> 0.39 ms at
@@ -601,35 +600,14 @@ static int fetch_rows(hg_ctx *c, const double *src, long len, long nrow, Take ta
                           hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipEventRecord(c->stage_ev[q], c->stream));
   }
-  // chunks [0, ready) have arrived; nchunk + 1 tells the helpers to give up
-  std::atomic<long> ready{0}, next{0};
-  auto hand_over = [&](long q) {
-    const long r1 = std::min(nrow, (q + 1) * rows);
-    for (long r = q * rows; r < r1; ++r) take(r);
-  };
-  auto help = [&] {
-    for (long q; (q = next.fetch_add(1)) < nchunk;) {
-      long got;
-      while ((got = ready.load(std::memory_order_acquire)) <= q) std::this_thread::yield();
-      if (got > nchunk) return;
-      hand_over(q);
-    }
-  };
   const long cpus = (long)std::thread::hardware_concurrency();
-  const long helpers = std::min({MAX_THREADS, cpus, nchunk / 2}) - 1;
-  std::thread th[MAX_THREADS];
-  long nth = 0;
-  try {
-    for (; nth < helpers; ++nth) th[nth] = std::thread(help);
-  } catch (const std::system_error &) {  // fewer threads: the caller does the rest
-  }
-  bool ok = true;
-  for (long q = 0; q < nchunk && ok; ++q) {
-    ok = hipEventSynchronize(c->stage_ev[q]) == hipSuccess;
-    ready.store(ok ? q + 1 : nchunk + 1, std::memory_order_release);
-  }
-  if (ok) help();
-  for (long q = 0; q < nth; ++q) th[q].join();
+  const bool ok = hand_over_chunks(
+      nchunk, std::min({MAX_THREADS, cpus, nchunk / 2}) - 1,
+      [&](long q) { return hipEventSynchronize(c->stage_ev[q]) == hipSuccess; },
+      [&](long q) {
+        const long r1 = std::min(nrow, (q + 1) * rows);
+        for (long r = q * rows; r < r1; ++r) take(r);
+      });
   return ok ? HG_OK : HG_ERR_DEVICE;
 }
 
