@@ -59,6 +59,14 @@ struct hg_ctx {
   // its own W fields these (d, e, B alias U as in the other sets)
   double *alt2_W[NWMAX] = {};
   bool alt2_ready = false;
+  // the further sets' own allocations, and the arrays hg_create made, where the
+  // state returns to when they are given back (drop_sets)
+  void *alt_mem = nullptr, *alt2_mem = nullptr;
+  StateSet base = {};
+  double *base_U0[NVMAX] = {};
+  // held by every call that uses the state, so that no other thread takes the
+  // further sets back meanwhile (take_back)
+  mutable std::mutex use;
   bool in_batch = false;
   // the batch it is in, and its three state sets as the batch's device
   // records number them (set 0 is the one D held when they were built)
@@ -80,8 +88,61 @@ static const char kVersion[] = "hormone_hip 0.1 (gfx950)";
 
 extern "C" const char *hg_version(void) { return kVersion; }
 
+using Use = std::lock_guard<std::mutex>;
+
+// Contexts whose further state sets may be taken back: those that took them by
+// themselves (default_form), as long as they are in no batch.  Memory that a
+// context may do without must not make another allocation of this library
+// fail.  Lock order: mu, then a context's use.
+struct Lenders {
+  std::mutex mu;
+  std::vector<hg_ctx *> list;
+};
+static Lenders &lenders() {
+  static Lenders *l = new Lenders;  // contexts may outlive static objects
+  return *l;
+}
+static void claim_sets(hg_ctx *c) {
+  Lenders &l = lenders();
+  const Use lock(l.mu);
+  l.list.erase(std::remove(l.list.begin(), l.list.end(), c), l.list.end());
+}
+static void lend_sets(hg_ctx *c) {
+  if (!c->alt_ready || !c->auto_form || c->in_batch) return;
+  Lenders &l = lenders();
+  const Use lock(l.mu);
+  if (std::find(l.list.begin(), l.list.end(), c) == l.list.end()) l.list.push_back(c);
+}
+static int drop_sets(hg_ctx *c);
+
+// Frees one lender's sets on this device; false if there is none.
+static bool take_back(int device) {
+  Lenders &l = lenders();
+  const Use lock(l.mu);
+  for (size_t q = 0; q < l.list.size(); ++q) {
+    hg_ctx *c = l.list[q];
+    if (c->device != device) continue;
+    const Use busy(c->use);  // a call in progress ends first
+    l.list.erase(l.list.begin() + q--);
+    if (drop_sets(c) == HG_OK) return true;
+  }
+  return false;
+}
+
+// On the current device.
+static int dev_malloc(size_t bytes, void **p) {
+  int device = 0;
+  HIPCHK(hipGetDevice(&device));
+  while (hipMalloc(p, bytes) != hipSuccess) {
+    (void)hipGetLastError();  // kept by HIP, and no error of a later launch
+    *p = nullptr;
+    if (!take_back(device)) return HG_ERR_NOMEM;
+  }
+  return HG_OK;
+}
+
 static int dev_alloc(hg_ctx *c, size_t bytes, void **p) {
-  if (hipMalloc(p, bytes) != hipSuccess) return HG_ERR_NOMEM;
+  if (int st = dev_malloc(bytes, p)) return st;
   c->allocs.push_back(*p);
   return HG_OK;
 }
@@ -94,11 +155,15 @@ static int dev_alloc(hg_ctx *c, size_t bytes, void **p) {
 // FP32-mixed 4,409 -> 4,012 (256 bytes and 4.25 KB apart: the same).  It is also
 // one allocation instead of up to 45 (hg_create and hg_destroy of a 97x131x75
 // MHD box 17.3 -> 1.0 ms).
+static size_t field_pitch(size_t bytes) { return (bytes + 4095) / 4096 * 4096 + 1024; }
+static void place_fields(void *mem, const std::vector<double **> &slot, size_t bytes) {
+  for (size_t q = 0; q < slot.size(); ++q)
+    *slot[q] = reinterpret_cast<double *>(static_cast<char *>(mem) + q * field_pitch(bytes));
+}
 static int dev_fields(hg_ctx *c, const std::vector<double **> &slot, size_t bytes) {
-  const size_t pitch = (bytes + 4095) / 4096 * 4096 + 1024;
-  char *p = nullptr;
-  if (int st = dev_alloc(c, pitch * slot.size(), (void **)&p)) return st;
-  for (size_t q = 0; q < slot.size(); ++q) *slot[q] = reinterpret_cast<double *>(p + q * pitch);
+  void *p = nullptr;
+  if (int st = dev_alloc(c, field_pitch(bytes) * slot.size(), &p)) return st;
+  place_fields(p, slot, bytes);
   return HG_OK;
 }
 
@@ -156,7 +221,7 @@ static int validate(const hg_desc *d) {
 static bool fused_now(const hg_ctx *c) { return c->fused && !c->in_batch; }
 
 static int fused_direction(const hg_ctx *c, int32_t on);
-static int ensure_fused_buffers(hg_ctx *c, int L);
+static int ensure_fused_buffers(hg_ctx *c, int L, bool spare = false);
 
 // The form a context starts with (hg_set_fused changes it; the results are the
 // same bits).  1D boxes: their one direction is fused, a stage is then one
@@ -167,25 +232,17 @@ static int ensure_fused_buffers(hg_ctx *c, int L);
 // 97x131x75 978 -> 632, 160^3 hydro 1333 -> 979); below, the one launch for
 // all directions does (160^2 59 against 61, 48^3 even, 40^3 90 against 114).
 // Without x (a y-z plane) the separate form is faster (512^2: 264 against 530).
-// A box whose further state sets do not fit keeps the separate form.
+// A box whose further state sets would leave less than an eighth of the GPU's
+// memory free keeps the separate form (the runtime too needs some, for queues
+// and scratch), and one that has them returns to it when their memory is needed
+// (take_back).
 static void default_form(hg_ctx *c) {
   const Dev &D = c->D;
   const int on = D.dim == 1 ? (D.solve[0] ? 2 : 1) : 2;
   if (D.dim == 0 || (D.dim == 2 && D.ncell < 1 << 15) || (D.dim == 3 && D.ncell < 1 << 17)) return;
   const int L = fused_direction(c, on);
   if (L < 0) return;
-  const size_t held = c->allocs.size();
-  double *const part = D.part;
-  const long cap = c->part_cap;
-  if (ensure_fused_buffers(c, L) != HG_OK) {
-    (void)hipGetLastError();
-    for (size_t q = held; q < c->allocs.size(); ++q) hipFree(c->allocs[q]);
-    c->allocs.resize(held);
-    c->alt_ready = c->alt2_ready = false;
-    c->D.part = part;
-    c->part_cap = cap;
-    return;
-  }
+  if (ensure_fused_buffers(c, L, true) != HG_OK) return;
   c->D.fdir = L;
   c->fused = true;
 }
@@ -444,13 +501,20 @@ extern "C" int hg_create(const hg_desc *desc, hg_ctx **out) {
       D.grav ? sizeof(double) * (size_t)(D.n1 + 2) * (D.n2 + 2) * (D.n3 + 2) : fb;
   if (hipHostMalloc((void **)&c->h_stage, stage, hipHostMallocDefault) != hipSuccess)
     return fail(HG_ERR_NOMEM);
+  for (int v = 0; v < D.nv; ++v) {
+    c->base.U[v] = D.U[v];
+    c->base_U0[v] = D.U0[v];
+  }
+  for (int w = 0; w < D.nw; ++w) c->base.W[w] = D.W[w];
   default_form(c);
+  lend_sets(c);
   *out = c;
   return HG_OK;
 }
 
 extern "C" int hg_destroy(hg_ctx *c) {
   if (!c) return HG_OK;
+  claim_sets(c);
   hipSetDevice(c->device);
   if (c->stream) hipStreamSynchronize(c->stream);
   if (c->gstream) hipStreamSynchronize(c->gstream);
@@ -459,6 +523,8 @@ extern "C" int hg_destroy(hg_ctx *c) {
   if (c->gdone) hipEventDestroy(c->gdone);
   if (c->gstream) hipStreamDestroy(c->gstream);
   for (void *p : c->allocs) hipFree(p);
+  if (c->alt_mem) hipFree(c->alt_mem);
+  if (c->alt2_mem) hipFree(c->alt2_mem);
   if (c->h_sc) hipHostFree(c->h_sc);
   if (c->h_stage) hipHostFree(c->h_stage);
   if (c->stream) hipStreamDestroy(c->stream);
@@ -512,6 +578,7 @@ static int batch_member_current(hg_ctx *c);
 
 extern "C" int hg_upload(hg_ctx *c, int32_t field, const double *a) {
   if (!c || !a) return HG_ERR_ARG;
+  const Use busy(c->use);
   if (int st = batch_member_current(c)) return st;
   if (field == HG_F_GRVPHI || field == HG_F_GRVPSI) {
     if (!c->D.grav) return HG_ERR_ARG;
@@ -613,6 +680,7 @@ static int fetch_rows(hg_ctx *c, const double *src, long len, long nrow, Take ta
 
 extern "C" int hg_download(hg_ctx *c, int32_t field, double *a) {
   if (!c || !a) return HG_ERR_ARG;
+  const Use busy(c->use);
   if (int st = batch_member_current(c)) return st;
   HIPCHK(hipSetDevice(c->device));
   const Dev &D = c->D;
@@ -738,6 +806,7 @@ static bool conserved_stages(const Dev &D) {
 extern "C" int hg_profile_read(const hg_ctx *c, int32_t kind, double *ms_total,
                                int64_t *launches, double *bytes_per_launch) {
   if (!c || kind < 0 || kind >= HG_PROF_N) return HG_ERR_ARG;
+  const Use busy(c->use);
   const Dev &D = c->D;
   const double cell = (double)D.ncell * sizeof(double);
   // the W fields that are not U (d, e and B alias U)
@@ -798,6 +867,7 @@ extern "C" int hg_profile_read(const hg_ctx *c, int32_t kind, double *ms_total,
 // stop flag is lifted for the replay and put back.
 extern "C" int hg_time_sweep(hg_ctx *c, int32_t launches, double *ms_total) {
   if (!c || launches <= 0 || !ms_total) return HG_ERR_ARG;
+  const Use busy(c->use);
   HIPCHK(hipSetDevice(c->device));
   int stop = 0;
   int *dstop = &c->D.sc->stop;
@@ -835,6 +905,7 @@ extern "C" int hg_timestep(hg_ctx *c, double time, double t_out, double t_end,
                            int32_t outstyle, int32_t endstyle, double fixed_dt, double *dt_out,
                            double *ch_out, double *cgrav_out, double *dtgrav_out) {
   if (!c) return HG_ERR_ARG;
+  const Use busy(c->use);
   HIPCHK(hipSetDevice(c->device));
   if (fixed_dt > 0.0) {
     if (dt_out) *dt_out = fixed_dt;
@@ -905,6 +976,7 @@ static void grav_speeds(const hg_ctx *c, double dt, double cfmax, double *cgrav,
 extern "C" int hg_gravity(hg_ctx *c, double time, double dt, double *grvtime, double cgrav,
                           double *cgrav_old, double *dtgrav, int32_t *nsub) {
   if (!c || !grvtime || !cgrav_old || !dtgrav) return HG_ERR_ARG;
+  const Use busy(c->use);
   if (!c->D.grav) return HG_ERR_STATE;
   HIPCHK(hipSetDevice(c->device));
   int st = ensure_eint(c);
@@ -1025,6 +1097,7 @@ static int enqueue_stages(hg_ctx *c, bool fuse_tail, double damp, bool sweep1_do
 
 extern "C" int hg_hydro_step(hg_ctx *c, double dt, double ch) {
   if (!c) return HG_ERR_ARG;
+  const Use busy(c->use);
   HIPCHK(hipSetDevice(c->device));
   int st = ensure_eint(c);
   if (st) return st;
@@ -1038,6 +1111,7 @@ extern "C" int hg_hydro_step(hg_ctx *c, double dt, double ch) {
 
 extern "C" int hg_phidamp(hg_ctx *c, double factor) {
   if (!c) return HG_ERR_ARG;
+  const Use busy(c->use);
   if (!c->D.mag) return HG_OK;
   HIPCHK(hipSetDevice(c->device));
   launch_phidamp(c->D, factor, c->stream);
@@ -1051,6 +1125,7 @@ extern "C" int hg_run(hg_ctx *c, double *time, int64_t *tn, double *t_out, doubl
                       int64_t tn_out, int64_t max_steps, double damp_factor,
                       int32_t *stop_reason) {
   if (!c || !time || !tn || !t_out || max_steps < 1) return HG_ERR_ARG;
+  const Use busy(c->use);
   if (outstyle == 2 && tn_out < 1) return HG_ERR_ARG;
   if (c->D.grav) return HG_ERR_UNSUPPORTED;  // gravity runs use hg_run_gravity
   HIPCHK(hipSetDevice(c->device));
@@ -1130,6 +1205,7 @@ extern "C" int hg_run_gravity(hg_ctx *c, double *time, int64_t *tn, double *t_ou
                               int64_t *nsub_total, int32_t *stop_reason) {
   if (!c || !time || !tn || !t_out || !grvtime || !cgrav_old || max_steps < 1)
     return HG_ERR_ARG;
+  const Use busy(c->use);
   if (outstyle == 2 && tn_out < 1) return HG_ERR_ARG;
   if (!c->D.grav) return HG_ERR_STATE;
   HIPCHK(hipSetDevice(c->device));
@@ -1280,43 +1356,93 @@ static bool own_field(const Dev &D, int w) {  // W fields a further set holds it
 // alias U in every set, as in hg_create; a phi the update does not write,
 // 1D MHD, is shared) and one CFL partial per block of direction L's fused
 // launch (one wavefront per block at most).
-static int ensure_fused_buffers(hg_ctx *c, int L) {
+// All of them or none.  spare: only where the GPU keeps memory to spare.
+static int ensure_fused_buffers(hg_ctx *c, int L, bool spare) {
   Dev &D = c->D;
-  if (!c->alt_ready) {
-    std::vector<double **> slot;
-    for (int v = 0; v < D.nv; ++v) slot.push_back(&c->alt_U[v]);
-    for (int w = 0; w < D.nw; ++w)
-      if (own_field(D, w)) slot.push_back(&c->alt_W[w]);
-    if (int st = dev_fields(c, slot, sizeof(double) * (size_t)D.ncell)) return st;
-    for (int w = 0; w < D.nw; ++w) {
-      if (w == WD) c->alt_W[w] = c->alt_U[0];
-      else if (w == WE) c->alt_W[w] = c->alt_U[4];
-      else if (D.mag && w >= WB1 && w <= WB3) c->alt_W[w] = c->alt_U[5 + (w - WB1)];
-      else if (w == WPHI && D.i9wv < 0) c->alt_W[w] = D.W[w];
+  const size_t fb = sizeof(double) * (size_t)D.ncell;
+  auto get = [&](size_t bytes, void **p) -> int {
+    size_t left = 0, total = 0;
+    if (!spare) return dev_malloc(bytes, p);
+    if (hipMemGetInfo(&left, &total) == hipSuccess && left >= bytes + total / 8 &&
+        hipMalloc(p, bytes) == hipSuccess)
+      return HG_OK;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return HG_ERR_NOMEM;
+  };
+  std::vector<double **> slot, slot2;
+  for (int v = 0; v < D.nv; ++v) slot.push_back(&c->alt_U[v]);
+  for (int w = 0; w < D.nw; ++w)
+    if (own_field(D, w)) {
+      slot.push_back(&c->alt_W[w]);
+      slot2.push_back(&c->alt2_W[w]);
     }
+  void *m1 = nullptr, *m2 = nullptr, *part = nullptr;
+  int st = HG_OK;
+  if (!c->alt_ready) st = get(field_pitch(fb) * slot.size(), &m1);
+  if (!st && !c->alt2_ready) st = get(field_pitch(fb) * slot2.size(), &m2);
+  if (!st && D.waves[L] > c->part_cap) st = get(sizeof(double) * 2 * (size_t)D.waves[L], &part);
+  if (st) {
+    for (void *p : {m1, m2, part})
+      if (p) (void)hipFree(p);
+    return st;
+  }
+  // the W fields of a further set that are its U, or, a phi nothing updates,
+  // every set's
+  auto alias = [&](double **W, double *const *U) {
+    W[WD] = U[0];
+    W[WE] = U[4];
+    for (int w = WB1; D.mag && w <= WB3; ++w) W[w] = U[5 + (w - WB1)];
+    if (D.mag && D.i9wv < 0) W[WPHI] = D.W[WPHI];
+  };
+  if (m1) {
+    place_fields(m1, slot, fb);
+    alias(c->alt_W, c->alt_U);
+    c->alt_mem = m1;
     c->alt_ready = true;
   }
-  if (D.waves[L] > c->part_cap) {
-    double *p = nullptr;
-    int st = dev_alloc(c, sizeof(double) * 2 * (size_t)D.waves[L], (void **)&p);
-    if (st) return st;
-    D.part = p;
-    c->part_cap = D.waves[L];
-  }
   // the third state set: U is D.U0's arrays, W its own fields
-  if (!c->alt2_ready) {
-    std::vector<double **> slot;
-    for (int w = 0; w < D.nw; ++w)
-      if (own_field(D, w)) slot.push_back(&c->alt2_W[w]);
-    if (int st = dev_fields(c, slot, sizeof(double) * (size_t)D.ncell)) return st;
-    for (int w = 0; w < D.nw; ++w) {
-      if (w == WD) c->alt2_W[w] = D.U0[0];
-      else if (w == WE) c->alt2_W[w] = D.U0[4];
-      else if (D.mag && w >= WB1 && w <= WB3) c->alt2_W[w] = D.U0[5 + (w - WB1)];
-      else if (w == WPHI && D.i9wv < 0) c->alt2_W[w] = D.W[w];
-    }
+  if (m2) {
+    place_fields(m2, slot2, fb);
+    alias(c->alt2_W, D.U0);
+    c->alt2_mem = m2;
     c->alt2_ready = true;
   }
+  if (part) {
+    c->allocs.push_back(part);
+    D.part = static_cast<double *>(part);
+    c->part_cap = D.waves[L];
+  }
+  return HG_OK;
+}
+
+// Gives the further sets' memory back: the state returns to the arrays
+// hg_create made, and the context to the separate form.  The caller sees to
+// it that no call and no batch uses the context.
+static int drop_sets(hg_ctx *c) {
+  if (!c->alt_ready && !c->alt2_ready) return HG_OK;
+  Dev &D = c->D;
+  HIPCHK(hipSetDevice(c->device));
+  for (int v = 0; v < D.nv; ++v)
+    if (D.U[v] != c->base.U[v]) launch_copy(D.U[v], c->base.U[v], D.ncell, c->stream);
+  for (int w = 0; w < D.nw; ++w)
+    if (own_field(D, w) && D.W[w] != c->base.W[w])
+      launch_copy(D.W[w], c->base.W[w], D.ncell, c->stream);
+  bool ok = hipGetLastError() == hipSuccess;
+  ok = hipStreamSynchronize(c->stream) == hipSuccess && ok;
+  if (c->gstream) ok = hipStreamSynchronize(c->gstream) == hipSuccess && ok;
+  if (!ok) return HG_ERR_DEVICE;
+  for (int v = 0; v < D.nv; ++v) {
+    D.U[v] = c->base.U[v];
+    D.U0[v] = c->base_U0[v];
+  }
+  for (int w = 0; w < D.nw; ++w) D.W[w] = c->base.W[w];
+  c->fused = false;
+  D.fdir = -1;
+  (void)hipFree(c->alt_mem);
+  (void)hipFree(c->alt2_mem);
+  c->alt_mem = c->alt2_mem = nullptr;
+  c->alt_ready = c->alt2_ready = false;
   return HG_OK;
 }
 
@@ -1376,15 +1502,20 @@ extern "C" int hg_set_fused(hg_ctx *c, int32_t on) {
   HIPCHK(hipStreamSynchronize(c->stream));
   Dev &D = c->D;
   if (!on) {
+    claim_sets(c);
     c->fused = c->auto_form = false;
     D.fdir = -1;
-    return HG_OK;
+    return c->in_batch ? HG_OK : drop_sets(c);
   }
   if (on != 1 && on != 2) return HG_ERR_ARG;
   const int L = fused_direction(c, on);
   if (L < 0 || c->in_batch) return HG_ERR_UNSUPPORTED;
+  claim_sets(c);
   int st = ensure_fused_buffers(c, L);
-  if (st) return st;
+  if (st) {
+    lend_sets(c);
+    return st;
+  }
   D.fdir = L;
   c->fused = true;
   c->auto_form = false;
@@ -1413,8 +1544,8 @@ extern "C" int hg_kat(int32_t which, int32_t n, const double *in, double *out) {
   double *din = nullptr, *dout = nullptr;
   const size_t bi = sizeof(double) * (size_t)n * kat_nin[w];
   const size_t bo = sizeof(double) * (size_t)n * kat_nout[w];
-  if (hipMalloc((void **)&din, bi) != hipSuccess) return HG_ERR_NOMEM;
-  if (hipMalloc((void **)&dout, bo) != hipSuccess) {
+  if (dev_malloc(bi, (void **)&din)) return HG_ERR_NOMEM;
+  if (dev_malloc(bo, (void **)&dout)) {
     hipFree(din);
     return HG_ERR_NOMEM;
   }
@@ -1536,6 +1667,7 @@ extern "C" int hg_batch_destroy(hg_batch *b) {
   for (hg_ctx *c : b->members) {  // ordinary contexts again
     c->in_batch = false;
     c->batch = nullptr;
+    lend_sets(c);
   }
   if (b->d_bpar) hipFree(b->d_bpar);
   hipStreamDestroy(b->stream);
@@ -1576,9 +1708,14 @@ extern "C" int hg_batch_add(hg_batch *b, hg_ctx *c, double time, double t_out, d
   HIPCHK(hipSetDevice(b->device));
   int st = batch_hsc_reserve(b, b->members.size() + 1);
   if (st) return st;
+  claim_sets(c);  // from here on they are the batch's to use
   st = ensure_eint(c);
-  if (st) return st;
-  HIPCHK(hipStreamSynchronize(c->stream));
+  if (!st && hipStreamSynchronize(c->stream) != hipSuccess) st = HG_ERR_DEVICE;
+  if (!st && !b->want_fused && c->auto_form) st = drop_sets(c);
+  if (st) {
+    lend_sets(c);
+    return st;
+  }
   // the box's clock and its first CFL partials, on the batch stream
   launch_set_clock(c->D, time, t_out, t_end, dt_out, outstyle, endstyle, 0, tnlim,
                    tn_out < 1 ? 1 : tn_out, (long long)1 << 62, b->stream);
@@ -1608,6 +1745,7 @@ extern "C" int hg_batch_remove(hg_batch *b, hg_ctx *c) {
       b->sc_valid.erase(b->sc_valid.begin() + q);
       c->in_batch = false;
       c->batch = nullptr;
+      lend_sets(c);
       // keep the cached member states aligned with the member list (the
       // array holds a record per member since hg_batch_add)
       for (size_t r = q; r < b->members.size(); ++r) b->h_sc[r] = b->h_sc[r + 1];
@@ -1623,7 +1761,7 @@ static int grow(T **p, size_t *cap, size_t need) {
   if (*p) hipFree(*p);
   *p = nullptr;
   size_t n = need + need / 2 + 16;
-  if (hipMalloc((void **)p, n * sizeof(T)) != hipSuccess) return HG_ERR_NOMEM;
+  if (dev_malloc(n * sizeof(T), (void **)p)) return HG_ERR_NOMEM;
   *cap = n;
   return HG_OK;
 }
@@ -1668,8 +1806,11 @@ static int batch_rebuild(hg_batch *b) {
   // the x-fused form when every member sweeps x
   bool fused = b->want_fused && nb > 0 && b->rktype <= 3;
   for (hg_ctx *c : b->members) fused = fused && c->D.waves[0] > 0;
-  for (size_t q = 0; fused && q < nb; ++q)
-    if ((st = ensure_fused_buffers(b->members[q], 0))) return st;
+  if (!fused) HIPCHK(hipStreamSynchronize(b->stream));  // hg_batch_add's reductions
+  for (hg_ctx *c : b->members) {
+    st = fused ? ensure_fused_buffers(c, 0) : (c->auto_form ? drop_sets(c) : HG_OK);
+    if (st) return st;
+  }
   std::vector<Dev> boxes(fused ? 9 * nb : nb);
   std::vector<int2> si, ci;
   for (size_t q = 0; q < nb; ++q) {

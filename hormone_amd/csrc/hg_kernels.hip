@@ -2233,6 +2233,19 @@ __global__ void k_geo(Axis A, double2 *geo) {
   }
 }
 
+// One field onto another.  The pointers go in a record: HIP keeps what a
+// stream's last command names allocated, by a launch's pointer arguments too,
+// and `from` may be freed next.
+struct CopyArgs {
+  const double *from;
+  double *to;
+  long n;
+};
+__global__ __launch_bounds__(256) void k_copy(CopyArgs a) {
+  const long m = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (m < a.n) gptr(a.to)[m] = gptr(a.from)[m];
+}
+
 __global__ void k_clear_error(Scalars *sc) { sc->err = NOERR; }
 
 // dt, ch and the error status of a finished CFL reduction into a caller's
@@ -2439,6 +2452,10 @@ void launch_pressure(const Dev &D, hipStream_t s) {
 
 void launch_geo(const Axis &A, double2 *geo, hipStream_t s) {
   k_geo<<<nblk(A.n + 4, 256), 256, 0, s>>>(A, geo);
+}
+
+void launch_copy(const double *from, double *to, long n, hipStream_t s) {
+  k_copy<<<nblk(n, 256), 256, 0, s>>>(CopyArgs{from, to, n});
 }
 
 void launch_clear_error(const Dev &D, hipStream_t s) { k_clear_error<<<1, 1, 0, s>>>(D.sc); }

@@ -188,6 +188,7 @@ void runge_coeff(int stage, int rktype, double *faco, double *fact, double *facn
 
 void launch_pressure(const Dev &D, hipStream_t s);
 void launch_geo(const Axis &A, double2 *geo, hipStream_t s);  // fills A's geo table
+void launch_copy(const double *from, double *to, long n, hipStream_t s);
 void launch_clear_error(const Dev &D, hipStream_t s);
 void launch_timestep_out(const Dev &D, double *out, hipStream_t s);  // dt, ch, status
 void launch_set_step(const Dev &D, double dt, double ch, hipStream_t s);

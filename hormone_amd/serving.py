@@ -121,12 +121,12 @@ def setup(req: Request):
 
 def device_bytes(req: Request, batch_fused: bool = True) -> int:
     """HBM footprint of one MHD context: the 5 W fields that do not alias U,
-    U 9, U0 9, DU dim*9, and in an x-fused batch, or in a box that is fused
-    from the start (hg_create, by its size), the second state set (U 9, W 5)
-    and the third set's own W fields (5; its U is U0's arrays)."""
+    U 9, U0 9, DU dim*9, and in an x-fused batch the second state set (U 9,
+    W 5) and the third set's own W fields (5; its U is U0's arrays).  The sets
+    a context takes by itself at the start are not counted: a separate batch
+    gives them back, and so does the library when memory runs short."""
     nv = 9
-    sets = batch_fused or req.cells >= (1 << 15 if req.dim == 2 else 1 << 17)
-    return 8 * req.cells * (5 + 2 * nv + req.dim * nv + (nv + 10 if sets else 0)) + \
+    return 8 * req.cells * (5 + 2 * nv + req.dim * nv + (nv + 10 if batch_fused else 0)) + \
         (1 << 20)
 
 

@@ -272,10 +272,14 @@ int hg_set_boundary_flux(hg_ctx *ctx, int32_t face, const double *flux);
    divergence is never written to or read back from HBM; the other
    directions are swept first.  Results are bit-identical either way, in
    FP64 and FP32-mixed.  Not with species, boundary codes 4, 5, 9, 10 or
-   while the context is in a batch (HG_ERR_UNSUPPORTED).  A context that
-   starts separate allocates the further copies of the state at the first
-   call (the launch reads one and writes another).  No counterpart in the
-   reference (a launch-shape choice). */
+   while the context is in a batch (HG_ERR_UNSUPPORTED).
+   A fused launch reads one copy of the state and writes another: the form
+   holds 19 fields for MHD and 13 for hydro beside the 50 and 29 of a
+   separate 3D context.  on = 0 gives them back.  A context takes them by
+   itself only where an eighth of the GPU's memory stays free, and loses them
+   again, with the same results in the separate form, when another allocation
+   of this library on the device would fail otherwise; for the memory of others
+   call with 0.  No counterpart in the reference (a launch-shape choice). */
 int hg_set_fused(hg_ctx *ctx, int32_t on);
 
 /* The sweep kernel's duration without per-dispatch events: `launches`
