@@ -92,6 +92,7 @@ __device__ __forceinline__ int wave_kept() {
 
 struct Cell {
   double d, v[3], e, eint, b[3], phi;
+  int mlow = 0;  // of cons_prims
 };
 
 __device__ __forceinline__ int ghost_src(int code, bool lo, int c, int n) {
@@ -153,9 +154,11 @@ __device__ __forceinline__ Cell finish_cell(const Dev &D, const Axis &A, int c,
 // The conserved state D.U holds between the stages of a fused step (Dev::cons):
 // from d, m, e and B of a cell to its velocities and internal energy, as the RK
 // update computes them (rk_cell_rt).  FAST: without operand scaling; the
-// sweep's own tests cover it (Chk).
+// sweep's own tests cover it (Chk).  Returns the momenta's lowest exponent for
+// them (odd_cell).
 template <bool MAG, bool FAST>
-__device__ __forceinline__ void cons_prims(double f[NWMAX]) {
+__device__ __forceinline__ int cons_prims(double f[NWMAX]) {
+  const int mlow = FAST ? lowest(f[WV1], f[WV2], f[WV3]) : 0;
   if (FAST) {
     const Den64 d = fden(f[WD]);
 #pragma unroll
@@ -166,6 +169,7 @@ __device__ __forceinline__ void cons_prims(double f[NWMAX]) {
   }
   f[WEINT] = get_eint(MAG, f[WE], f[WD], f[WV1], f[WV2], f[WV3], MAG ? f[WB1] : 0.0,
                       MAG ? f[WB2] : 0.0, MAG ? f[WB3] : 0.0);
+  return mlow;
 }
 
 // where field w of the state is: momenta for velocities and U's psi if CONS
@@ -310,9 +314,12 @@ __device__ __forceinline__ Cell load_cell(const Dev &D, const Axis &A, long base
     for (int a = 0; a < 3; ++a) f[WB1 + a] = gptr(D.W[WB1 + a])[mv];
     f[WPHI] = gptr(state_field<CONS>(D, WPHI))[ms];
   }
-  if (CONS) cons_prims<MAG, FAST>(f);
+  int mlow = 0;
+  if (CONS) mlow = cons_prims<MAG, FAST>(f);
   else f[WEINT] = gptr(D.W[WEINT])[ms];
-  return finish_cell<DIR, MAG>(D, A, c, f);
+  Cell q = finish_cell<DIR, MAG>(D, A, c, f);
+  q.mlow = mlow;
+  return q;
 }
 
 // ---- LDS-staged lines for the strided (y, z) sweeps ------------------------
@@ -503,9 +510,12 @@ __device__ __forceinline__ Cell tile_column(const Dev &D, const Axis &A, int c,
   const double *p = lds + lane * ld + w;
 #pragma unroll
   for (int k = 0; k < NWMAX; ++k) f[k] = k < nf && k != WEINT ? p[k * fs] : 0.0;
-  if (CONS) cons_prims<MAG, FAST>(f);
+  int mlow = 0;
+  if (CONS) mlow = cons_prims<MAG, FAST>(f);
   else f[WEINT] = p[WEINT * fs];
-  return finish_cell<DIR, MAG>(D, A, c, f);
+  Cell q = finish_cell<DIR, MAG>(D, A, c, f);
+  q.mlow = mlow;
+  return q;
 }
 
 template <int DIR, bool MAG, bool EXT, bool CONS, bool FAST>
@@ -823,13 +833,14 @@ __device__ __forceinline__ Geo load_geo(const Axis &A, int c) {
 // Flux t of the face c+1/2 of every lane of a wavefront from the lanes' cells
 // (checked fast form).  True, for the whole wavefront, when one of its
 // faces -1 .. n-1 depends on a value out of the fast form's range.
-template <int DIR, bool MAG, int LIM>
+template <int DIR, bool MAG, int LIM, bool CONS>
 __device__ __forceinline__ bool line_faces(const Axis &A, const Cell &q, int c, int lane,
                                            double gam, const Den64 &Dch, double t[9]) {
   const int n = A.n;
   double qv[9], ql[9], qr[9];
   slope_values<MAG>(q, qv);
-  unsigned long long bad = __builtin_amdgcn_ballot_w64(odd_cell<MAG>(qv));
+  const int mlow = CONS ? q.mlow : lowest(qv[2], qv[3], qv[4]);
+  unsigned long long bad = __builtin_amdgcn_ballot_w64(odd_cell<MAG>(qv, mlow));
   if (LIM != LIM_FLAT) {
 #pragma unroll
     for (int s = 0; s < 9; ++s) {
@@ -901,6 +912,27 @@ __device__ __forceinline__ void line_faces_plain(const Axis &A, const Cell &q, i
   face_flux<DIR, MAG>(L, S, R_, RS, dx1, dx2, gam, ch, t, fe);
 }
 
+// Whether a cell this wavefront updates has a momentum of -0 (Chk: zeros), from
+// the tile or the parked cells, which hold its velocity or momentum.
+template <bool TILE, bool FUSED, bool CONS>
+__device__ __forceinline__ bool minus_zero(const Dev &D, const Axis &A, long base, int c,
+                                           const double *lds) {
+  const int lane = lane_again<TILE>();
+  bool z = false;
+  if (lane >= 2 && lane <= 61 && c >= 0 && c < A.n) {
+    const int bw = blockDim.x >> 6, ld = tile_ld(bw), w = wave_in_block();
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      double m;
+      if (TILE) m = lds[(WV1 + a) * 64 * ld + lane * ld + w];
+      else if (FUSED) m = lds[(2 + a) * blockDim.x + lane];
+      else m = gptr(state_field<CONS>(D, WV1 + a))[base + (long)c * A.stride];
+      z |= __builtin_amdgcn_class(m, 0x20);
+    }
+  }
+  return __builtin_amdgcn_ballot_w64(z) != 0;
+}
+
 // RK update of the cells a fused sweep has just finished (defined with the RK
 // kernels below)
 template <int DIR, bool MAG, bool TILE>
@@ -937,7 +969,8 @@ __device__ __forceinline__ void sweep_line(const Dev &D, long wave, int lane, in
   const Den64 Dch{gptr(D.sc)->ch, gptr(D.sc)->chr};
   double t[9];
   bool neg = false;  // a face density or internal energy is not positive
-  const bool odd = line_faces<DIR, MAG, LIM>(A, q, c, lane, gam, Dch, t);
+  bool odd = line_faces<DIR, MAG, LIM, CONS>(A, q, c, lane, gam, Dch, t);
+  if (D.grav) odd = odd || minus_zero<TILE, FUSED, CONS>(D, A, (long)ubase, c, lds);
   // the rare branches place the lane again, so that nothing is kept for them
   auto again = [&](long &line2, long &base2, int &c2) {
     lane_cell<DIR>(D, A, wave, lane_again<TILE>(), line2, base2, c2);

@@ -293,23 +293,47 @@ __device__ __forceinline__ void hlld(R f[9], R cfl, R cfr, R v1l, R v1r, R v2l, 
 // launch) 594 -> 437 us.
 //
 // Chk: pos() takes a value that has to be positive with an exponent in
-// [-256, 255], neg() a negative one, num() one of either sign that may also be
-// zero (its frexp exponent is 0 then), differ() a pair whose order decides.
+// [-256, 255], neg() a negative one, leaf() one of either sign that is zero (its
+// frexp exponent is 0 then) or has an exponent of at least -600, num() (known-answer
+// records) one with an exponent in [-256, 255], differ() a pair whose order
+// decides.
 //
 // What is tested, and why it is enough.  A quotient or root without scaling is
 // exact unless its dividend or radicand is below 2^-968 (an inexact residual),
 // the divisor extreme, or the quotient overflows or is denormal.
-// * Every cell (odd_cell): d, e and e_int in range, so |m| <= 2^257 and |b| <=
-//   2^129; no NaN, infinity or -0.  Face densities and energies, the squared
+// * Every cell (odd_cell): d, e and e_int in range, which leaves no NaN or
+//   infinity in the velocities and fields they hold the energy of, |m| <= 2^257
+//   and |b| <= 2^129; m and b leaves.  Face densities and energies, the squared
 //   sound speeds, and every divisor and radicand of the solver: in range.  So
 //   no divisor is extreme and no quotient overflows.
-// * What is left are dividends that are tiny but not zero.  Their quotients are
-//   tiny too and wrong by an ulp at most.  Such a value is lost in a sum with
-//   any value in range, and the sums that always hold one need no test: the
-//   energies and pressures, the wave speeds (a fast speed is in range), pta.
-//   Where all of a sum may be tiny its result is tested: sm's dividend, b1,
-//   the face's psi and, for all that feeds them (the limited slopes, the
-//   velocities, the star states), the selected transverse velocity and field.
+// * Leaves make the face states exact.  Differences of neighbours are 0 or at
+//   least 2^-652; with the grid factors' ranges (Axis::fast) the limiters'
+//   dividends are then at least 2^-870 and their quotients 2^-970, so the
+//   slopes, the face momenta and fields (0 or above 2^-690) and their
+//   velocities are exact, and so is sm: -ptr + ptl leaves a dividend of 0 or of
+//   pt's last place (2^-567) or more.  psi has no slopes; dphi is a leaf.
+// * What is left are tiny dividends made of products.  Their quotients are
+//   below 2^-712 and wrong by an ulp at most.  Such a value is lost in a sum
+//   with any value in range: the energies and pressures, the wave speeds (a
+//   fast speed is in range), pta.  In a side's transverse star states it is
+//   tested for: the velocity or the dividend taken off it is a leaf (less()),
+//   and the fields' factor is 0 or has 2^-257 or more, so that their dividends
+//   are 0 or above 2^-947.  The inner states are made of these, with dividends
+//   of 0 or above 2^-900: exact as well, unless a star density is 2^279 times
+//   below its side's (a quotient could be denormal).
+// * Zeros may have the other sign: of a momentum or field of a ghost (a wall
+//   makes -0 of +0), and of slopes (vmin and vmax do not order zeros).  That
+//   reaches the fluxes as the sign of a zero only.  The selections are by sm
+//   and the Alfven speeds; sm's zero is +0 (x - ptr + ptl), and where b1 is a
+//   zero both Alfven speeds have sm's sign.  And an update shows no flux
+//   divergence's zero: with the source's +0 the sum is +0.  Only gravity's
+//   source may be -0, and only a momentum of -0 shows that (minus_zero).
+// A wavefront that runs both forms takes 1.7 (MHD) to 2 (hydro) times as long:
+// 56^3, three directions in one launch, every wavefront: 40 -> 70 us, 22 -> 44.
+// With every -0 refused, that was each wavefront at a wall of gas at rest, or of
+// zero normal field, or with inflow; with 2^-256 as the limit of what was tested,
+// up to 70% of an MHD blast wave's (96^3, 16 steps after the start: 846 us per
+// step, now 505), whose velocities fall off through that ahead of the front.
 // The tests are asm volatile so that each is made where its value is computed:
 // written as expressions they were gathered at the end of the block, with
 // every tested value kept in registers until then (162 VGPRs against 126; 102
@@ -323,6 +347,24 @@ struct Chk {
         "v_frexp_exp_i32_f64 %1, %2\n\tv_add_u32 %1, 0x100, %1\n\tv_or_b32 %0, %0, %1"
         : "+v"(n), "=&v"(t)
         : "v"(x));
+  }
+  template <int LOW = 600>
+  __device__ __forceinline__ void leaf(double x) {
+    unsigned t;
+    asm volatile(
+        "v_frexp_exp_i32_f64 %1, %2\n\tv_add_u32 %1, %3, %1\n\tv_or_b32 %0, %0, %1"
+        : "+v"(p), "=&v"(t)
+        : "v"(x), "i"(LOW));
+  }
+  // x = z - a/d: leaf() of the larger of x and a
+  __device__ __forceinline__ void less(double x, double a) {
+    double y;
+    unsigned t;
+    asm volatile(
+        "v_max_f64 %2, |%3|, |%4|\n\tv_frexp_exp_i32_f64 %1, %2\n\t"
+        "v_add_u32 %1, 0x258, %1\n\tv_or_b32 %0, %0, %1"
+        : "+v"(p), "=&v"(t), "=&v"(y)
+        : "v"(x), "v"(a));
   }
   __device__ __forceinline__ void pos(double x) { high<0xd0100000u>(__double2hiint(x)); }
   __device__ __forceinline__ void neg(double x) { high<0x50100000u>(__double2hiint(x)); }
@@ -358,7 +400,7 @@ __device__ __forceinline__ double fsqrt(double x) {
 }
 // min and max of two numbers, one instruction (the reference's a < b ? a : b
 // takes three; they differ for NaN, which the sweep's cells are tested for,
-// and in the sign of a zero, see cell_faces).  fmin() would add two
+// and in the sign of a zero, see Chk).  fmin() would add two
 // instructions that quiet signalling NaNs.
 __device__ __forceinline__ double vmin(double a, double b) {
   double r;
@@ -426,8 +468,7 @@ __device__ __forceinline__ double fslope(double u0, double u1, double u2, const 
 // guard's own face values are the Riemann states unless it resets the slopes
 // to zero (then they are the cell's value), so nothing is evaluated twice.
 //
-// odd_cell keeps out what vmin and vmax treat otherwise; a slope's zero may
-// have the other sign, which q +- h*S does not show where q is not -0.
+// vmin and vmax may give a slope's zero the other sign (Chk: zeros).
 template <bool MAG, int LIM>
 __device__ __forceinline__ void cell_faces(const double qv[9], const double ql[9],
                                            const double qr[9], const Geo &G, double FL[8],
@@ -474,19 +515,22 @@ __device__ __forceinline__ void cell_faces(const double qv[9], const double ql[9
   }
 }
 
-// A cell the fast form is not for: d, e or e_int out of range, or a momentum or
-// field that is NaN, infinite or -0 (vmin and vmax treat those otherwise than
-// the reference's comparisons).
+// The lowest exponent of three values, zeros (exponent 0) and those above 1 apart.
+__device__ __forceinline__ int lowest(double x, double y, double z) {
+  const int a = __builtin_amdgcn_frexp_exp(x), b = __builtin_amdgcn_frexp_exp(y),
+            c = __builtin_amdgcn_frexp_exp(z);
+  return min(min(a, b), c);
+}
+
+// A cell the fast form is not for: d, e or e_int out of range, or a momentum (the
+// lowest exponent mlow) or field that is no leaf.
 template <bool MAG>
-__device__ __forceinline__ bool odd_cell(const double qv[9]) {
+__device__ __forceinline__ bool odd_cell(const double qv[9], int mlow) {
   Chk k;
   k.pos(qv[0]);
   k.pos(qv[1]);
   k.pos(qv[8]);
-  bool b = k.bad();
-#pragma unroll
-  for (int s = 2; s < (MAG ? 8 : 5); ++s) b |= __builtin_amdgcn_class(qv[s], 0x227);
-  return b;
+  return k.bad() || min(mlow, MAG ? lowest(qv[5], qv[6], qv[7]) : 0) < -600;
 }
 
 // get_cf, the checked fast form
@@ -506,8 +550,8 @@ __device__ __forceinline__ double fast_cf(const Den64 &Dd, double cs, double b1,
 // reciprocal.  Hydro (MAG false): with B = 0 and psi = 0 the transverse
 // states, the Alfven states and every term with b1 are the identity or a
 // zero, and both Alfven speeds are sm, so only the contact's selection is
-// left; what changes is the sign of a zero flux, which no update of a state
-// without -0 shows.
+// left; what changes is the sign of a zero flux (Chk: zeros), and with exact
+// face states every value selected is exact.
 template <bool MAG>
 __device__ __forceinline__ void hlld_fast(double f[9], double cfl, double cfr, double v1l,
                                           double v1r, double v2l, double v2r, double v3l,
@@ -519,11 +563,9 @@ __device__ __forceinline__ void hlld_fast(double f[9], double cfl, double cfr, d
   const double ch = Dch.b;
   if constexpr (MAG) {  // first: psi and the sides' normal fields are done with then
     const double dphi = phir - phil;
-    k.num(dphi);
+    k.leaf(dphi);
     b1 = 0.5 * ((b1l + b1r) - fdiv_(Dch, dphi));
     phi = 0.5 * ((phil + phir) - (b1r - b1l) * ch);
-    k.num(b1);
-    k.num(phi);
     fence();
   }
   const double sl = vmin(vmin(v1r - cfr, v1l - cfl), 0.0);
@@ -534,7 +576,6 @@ __device__ __forceinline__ void hlld_fast(double f[9], double cfl, double cfr, d
   const Den64 Dden = fden(den);
   const double smn = srv * dr * v1r - slv * dl * v1l - ptr + ptl;
   const double pan = srv * dr * ptl - slv * dl * ptr + dl * dr * srv * slv * (v1r - v1l);
-  k.num(smn);
   const double sm = fdiv_(Dden, smn), pta = fdiv_(Dden, pan);
   const double slm = sl - sm, srm = sr - sm;
   k.neg(slm);
@@ -551,8 +592,6 @@ __device__ __forceinline__ void hlld_fast(double f[9], double cfl, double cfr, d
     const double wl = wpos(hsm), wr = wneg(hsm);
     const double d_ = wl * dla + wr * dra;
     const double v2_ = wl * v2l + wr * v2r, v3_ = wl * v3l + wr * v3r;
-    k.num(v2_);
-    k.num(v3_);
     f[0] = d_ * sm;
     f[1] = d_ * sm * sm + pta;
     f[2] = d_ * sm * v2_;
@@ -575,9 +614,12 @@ __device__ __forceinline__ void hlld_fast(double f[9], double cfl, double cfr, d
   const double dnl = dl * slv * slm - b1b1;
   k.pos(dnl);
   const Den64 Dl = fden(dnl);
-  const double v2la = v2l - fdiv_(Dl, b1 * b2l * (sm - v1l));
-  const double v3la = v3l - fdiv_(Dl, b1 * b3l * (sm - v1l));
+  const double a2l = b1 * b2l * (sm - v1l), a3l = b1 * b3l * (sm - v1l);
+  const double v2la = v2l - fdiv_(Dl, a2l), v3la = v3l - fdiv_(Dl, a3l);
+  k.less(v2la, a2l);
+  k.less(v3la, a3l);
   const double numl = dl * slv * slv - b1b1;
+  k.leaf<256>(numl);
   const double b2la = fdiv_(Dl, b2l * numl);
   const double b3la = fdiv_(Dl, b3l * numl);
   const double ela = fdiv_(Dslm, slv * el - ptl * v1l + pta * sm +
@@ -587,9 +629,12 @@ __device__ __forceinline__ void hlld_fast(double f[9], double cfl, double cfr, d
   const double dnr = dr * srv * srm - b1b1;
   k.pos(dnr);
   const Den64 Dr = fden(dnr);
-  const double v2ra = v2r - fdiv_(Dr, b1 * b2r * (sm - v1r));
-  const double v3ra = v3r - fdiv_(Dr, b1 * b3r * (sm - v1r));
+  const double a2r = b1 * b2r * (sm - v1r), a3r = b1 * b3r * (sm - v1r);
+  const double v2ra = v2r - fdiv_(Dr, a2r), v3ra = v3r - fdiv_(Dr, a3r);
+  k.less(v2ra, a2r);
+  k.less(v3ra, a3r);
   const double numr = dr * srv * srv - b1b1;
+  k.leaf<256>(numr);
   const double b2ra = fdiv_(Dr, b2r * numr);
   const double b3ra = fdiv_(Dr, b3r * numr);
   const double era = fdiv_(Dsrm, srv * er - ptr * v1r + pta * sm +
@@ -616,10 +661,6 @@ __device__ __forceinline__ void hlld_fast(double f[9], double cfl, double cfr, d
   const double v3_ = wl * v3la + wa * v3aa + wr * v3ra;
   const double b2_ = wl * b2la + wa * b2aa + wr * b2ra;
   const double b3_ = wl * b3la + wa * b3aa + wr * b3ra;
-  k.num(v2_);
-  k.num(v3_);
-  k.num(b2_);
-  k.num(b3_);
   const double e_ = wl * ela + wneg(hla ^ hsm) * elaa + wneg(hsm ^ hra) * eraa + wr * era;
   f[0] = d_ * sm;
   f[1] = d_ * sm * sm + pta - b1b1;
