@@ -787,11 +787,15 @@ extern "C" int hg_profile(hg_ctx *c, int32_t enable) {
 // reads.  Without them, with v and e_int computed by the sweeps that read the
 // state: fused sweep of 256^3 1,409 -> 1,246 us, y and z sweeps 1,684 -> 1,685,
 // 9,345 -> 8,850 us per step; 160^3 hydro 929 -> 875, 97x131x75 568 -> 538.
-// Boxes of up to 2^19 cells stay in the Infinity Cache and would only lose
-// (512^2 121.6 -> 123.8).  All fields are kept as well in boxes whose scalar and
-// vector boundary codes take a ghost from different cells, by the sweeps fused
-// along y or z, by FP32-mixed and in batches (1.5% for one of 1e6 cells, against
-// twice the kernels).
+// Boxes of up to 2^19 cells keep all fields: the gain grows with the launch and
+// is nothing at 2^18 (us per step without and with those fields: MHD 56^3 156.5,
+// 154.6; 64^3 186.6, 186.7; 512^2 123.9, 125.2; 81^3 312, 321; 1024^2 380, 405;
+// 128^3 1,156, 1,228).  The line is in cells for hydro too, which holds half the
+// bytes (64^3 119.5, 119.2; 81^3 191, 195; 1024^2 216, 229; 128^3 639, 701).
+// All fields are kept as well in boxes whose scalar and vector boundary codes
+// take a ghost from different cells, by the sweeps fused along y or z, by
+// FP32-mixed and in batches (1.5% for one of 1e6 cells, against twice the
+// kernels).
 static bool conserved_stages(const Dev &D) {
   auto source = [](int code) { return code < 2 ? code : 2; };  // as ghost_src
   bool one = D.fdir == 0 && !D.mixed && D.ncell > 1L << 19;

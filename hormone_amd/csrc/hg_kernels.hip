@@ -556,7 +556,7 @@ __device__ __forceinline__ Cell tile_cell(const Dev &D, const Axis &A, long wave
       const long ms = sv.x, mv = sv.y;
       p[WD * fs] = gptr(D.W[WD])[ms];
       p[WE * fs] = gptr(D.W[WE])[ms];
-          if (!CONS) p[WEINT * fs] = gptr(D.W[WEINT])[ms];
+      if (!CONS) p[WEINT * fs] = gptr(D.W[WEINT])[ms];
 #pragma unroll
       for (int a = 0; a < 3; ++a) p[(WV1 + a) * fs] = gptr(state_field<CONS>(D, WV1 + a))[mv];
       if (MAG) {
@@ -1512,9 +1512,10 @@ __device__ __forceinline__ void rk_cell_rt(const Dev &D, long m, int stage, doub
   double *const *Wo = LD >= 0 ? D.Wo : D.W;
   // Everything the update reads is loaded before anything is stored: the
   // stores might alias, and a load written after one waits for it, nine memory
-  // round trips in a row (@R@).  Two groups, the divergences and the states, as
-  // many as registers allow in flight; a psi that is not there reads B3 again,
-  // so that each group is straight code.
+  // round trips in a row (k_rk of 128^2 MHD 8.5 -> 6.4 us, 97x131x75 fused x
+  // sweep 84.7 -> 80.4, larger boxes even).  Two groups, the divergences and the
+  // states, as many as registers allow in flight; a psi that is not there reads
+  // B3 again, so that each group is straight code.
   const bool psi = MAG && D.nv == 9;
   constexpr int nv = MAG ? 9 : 5;
   auto load = [&](double *const *F, double x[NVMAX]) {
