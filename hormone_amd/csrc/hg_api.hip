@@ -138,6 +138,14 @@ static int dev_malloc(size_t bytes, void **p) {
     *p = nullptr;
     if (!take_back(device)) return HG_ERR_NOMEM;
   }
+  // The runtime needs some as well: the sweeps' scratch (about 20 MB for each of
+  // its queues) is allocated at a launch, and a launch that cannot have it ends
+  // the queue.
+  constexpr size_t RESERVE = 128 << 20;
+  size_t left = 0, total = 0;
+  while (bytes >= 1 << 20 && hipMemGetInfo(&left, &total) == hipSuccess && left < RESERVE &&
+         take_back(device)) {
+  }
   return HG_OK;
 }
 

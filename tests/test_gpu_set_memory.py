@@ -141,6 +141,28 @@ def test_gpu_separate_batch_gives_the_sets_back(hiplib, flow, separate, when):
     same(out[0], out[1])
 
 
+def test_gpu_sets_are_taken_back_before_memory_is_full(hiplib, flow, separate):
+    """An allocation that fits, but leaves the runtime next to nothing."""
+    need, three, five, mid, end = separate
+    hip, fill = native.lib(), C.c_void_p()
+    engs = [load(create(flow), flow)]
+    try:
+        assert run(engs[0], 0.0, 0, 3) == mid
+        assert hip.hipMalloc(C.byref(fill), C.c_size_t(free() - need - (64 << 20))) == 0
+        print("case a context that leaves 64 MiB", flush=True)
+        engs.append(load(create(flow), flow))
+        assert free() >= 0.9 * SETS
+        assert run(engs[1], 0.0, 0, 3) == mid
+        for eng in engs:
+            same(fields(eng, flow), three)
+            assert run(eng, *mid, 2) == end
+            same(fields(eng, flow), five)
+    finally:
+        for eng in engs:
+            eng.close()
+        assert hip.hipFree(fill) == 0
+
+
 @pytest.mark.parametrize("busy", [False, True], ids=["idle", "stepping"])
 def test_gpu_contexts_that_fit_without_the_sets_fit(hiplib, flow, separate, busy):
     """Two contexts with further sets, then memory for three more once one of
