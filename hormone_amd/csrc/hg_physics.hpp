@@ -287,10 +287,10 @@ __device__ __forceinline__ void hlld(R f[9], R cfl, R cfr, R v1l, R v1r, R v2l, 
 // computes its cells again with plain divisions and square roots
 // (cell_slopes, face_flux).  One test per face instead of a branch per
 // division leaves the compiler one straight block to schedule.  The y and z
-// sweeps are bound by VALU issue (about 85% busy), so this is their time:
-// 1,530 -> 1,124 VALU instructions per wavefront (256^3 MHD shear layer),
-// 2,075 -> 1,760 us per stage for both; hydro (160^3, three directions in one
-// launch) 594 -> 437 us.
+// sweeps are bound by VALU issue (78% busy with the quarter-rate reciprocals
+// counted as one), so this is their time: 1,530 -> 1,125 VALU instructions per
+// wavefront (256^3 MHD polytrope), 2,075 -> 1,760 us per stage for both (shear
+// layer); hydro (160^3, three directions in one launch) 594 -> 437 us.
 //
 // Chk: pos() takes a value that has to be positive with an exponent in
 // [-256, 255], neg() a negative one, leaf() one of either sign that is zero (its
