@@ -240,10 +240,9 @@ static int ensure_fused_buffers(hg_ctx *c, int L, bool spare = false);
 // 97x131x75 978 -> 632, 160^3 hydro 1333 -> 979); below, the one launch for
 // all directions does (160^2 59 against 61, 48^3 even, 40^3 90 against 114).
 // Without x (a y-z plane) the separate form is faster (512^2: 264 against 530).
-// A box whose further state sets would leave less than an eighth of the GPU's
-// memory free keeps the separate form (the runtime too needs some, for queues
-// and scratch), and one that has them returns to it when their memory is needed
-// (take_back).
+// A box whose further state sets would leave too little of the GPU's memory free
+// (ensure_fused_buffers) keeps the separate form, and one that has them returns
+// to it when their memory is needed (take_back).
 static void default_form(hg_ctx *c) {
   const Dev &D = c->D;
   const int on = D.dim == 1 ? (D.solve[0] ? 2 : 1) : 2;
@@ -1368,14 +1367,16 @@ static bool own_field(const Dev &D, int w) {  // W fields a further set holds it
 // alias U in every set, as in hg_create; a phi the update does not write,
 // 1D MHD, is shared) and one CFL partial per block of direction L's fused
 // launch (one wavefront per block at most).
-// All of them or none.  spare: only where the GPU keeps memory to spare.
+// All of them or none.  spare: only where the GPU keeps memory to spare, an eighth
+// of it or, for small boxes, sixteen times as much again and 256 MiB.
 static int ensure_fused_buffers(hg_ctx *c, int L, bool spare) {
   Dev &D = c->D;
   const size_t fb = sizeof(double) * (size_t)D.ncell;
   auto get = [&](size_t bytes, void **p) -> int {
     size_t left = 0, total = 0;
     if (!spare) return dev_malloc(bytes, p);
-    if (hipMemGetInfo(&left, &total) == hipSuccess && left >= bytes + total / 8 &&
+    if (hipMemGetInfo(&left, &total) == hipSuccess &&
+        left >= bytes + std::min(total / 8, 16 * bytes + ((size_t)256 << 20)) &&
         hipMalloc(p, bytes) == hipSuccess)
       return HG_OK;
     (void)hipGetLastError();

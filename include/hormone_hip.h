@@ -276,10 +276,12 @@ int hg_set_boundary_flux(hg_ctx *ctx, int32_t face, const double *flux);
    A fused launch reads one copy of the state and writes another: the form
    holds 19 fields for MHD and 13 for hydro beside the 50 and 29 of a
    separate 3D context.  on = 0 gives them back.  A context takes them by
-   itself only where an eighth of the GPU's memory stays free, and loses them
-   again, with the same results in the separate form, when another allocation
-   of this library on the device would fail otherwise or leave less than 128
-   MiB; for the memory of others call with 0.  No counterpart in the reference (a launch-shape choice). */
+   itself only where an eighth of the GPU's memory (or sixteen times their
+   size and 256 MiB, if that is less) stays free, and loses them again, with
+   the same results in the separate form, when another allocation of this
+   library on the device would fail otherwise or leave less than 128 MiB; for
+   the memory of others call with 0.  No counterpart in the reference (a
+   launch-shape choice). */
 int hg_set_fused(hg_ctx *ctx, int32_t on);
 
 /* The sweep kernel's duration without per-dispatch events: `launches`

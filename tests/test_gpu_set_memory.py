@@ -8,6 +8,7 @@ import threading
 import numpy as np
 import pytest
 
+import bench
 from hormone_amd import driver as D
 from hormone_amd import native
 from hormone_amd import problems as P
@@ -53,6 +54,13 @@ def create(flow):
 def load(eng, flow):
     D.load_initial_state(eng, *flow)
     return eng
+
+
+def form(eng, n, fused):
+    """Whether the context is in this form, by the bytes of its RK launch."""
+    cells, dim = n[0] * n[1] * n[2], sum(m > 1 for m in n)
+    want = bench.kernel_bytes(fused, eng.ufnmax(), 10, dim, True, 3, fused and cells > 1 << 19)[1]
+    return eng.profile_read(native.PROF_RK)[2] == pytest.approx(want * cells)
 
 
 def run(eng, t, tn, steps):
@@ -139,6 +147,21 @@ def test_gpu_separate_batch_gives_the_sets_back(hiplib, flow, separate, when):
         out.append(fields(eng, flow))
         eng.close()
     same(out[0], out[1])
+
+
+@pytest.mark.parametrize("n,fused", [((256, 256, 1), 2), ((1024, 1, 1), 2), (N, 0)])
+def test_gpu_sets_of_small_boxes_fit_where_large_ones_do_not(hiplib, flow, separate, n, fused):
+    """With 4 GiB left: the form a box starts with, by the bytes of its launches."""
+    hip, fill = native.lib(), C.c_void_p()
+    assert hip.hipMalloc(C.byref(fill), C.c_size_t(free() - (4 << 30))) == 0
+    try:
+        print(f"case form of {n} with 4 GiB left", flush=True)
+        prm = P.Params(n=n, mag_on=True, bc=(0,) * 12, is_test=False)
+        eng = Hydro(**D.desc_fields(prm, cartesian_grid(n, prm.lo, prm.hi)))
+        assert form(eng, n, fused)
+        eng.close()
+    finally:
+        assert hip.hipFree(fill) == 0
 
 
 def test_gpu_sets_are_taken_back_before_memory_is_full(hiplib, flow, separate):
