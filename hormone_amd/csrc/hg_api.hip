@@ -1652,6 +1652,15 @@ static int batch_member_current(hg_ctx *c) {
   return HG_OK;  // added since the last build: its state is in its own set
 }
 
+// An ordinary context again, in the form it starts with if it has not been
+// told otherwise (a separate batch has dropped its further sets).
+static void leave_batch(hg_ctx *c) {
+  c->in_batch = false;
+  c->batch = nullptr;
+  if (c->auto_form && !c->alt_ready) default_form(c);
+  lend_sets(c);
+}
+
 extern "C" int hg_batch_create(int32_t device, hg_batch **out) {
   if (!out) return HG_ERR_ARG;
   *out = nullptr;
@@ -1678,9 +1687,7 @@ extern "C" int hg_batch_destroy(hg_batch *b) {
   if (b->h_sc) hipHostFree(b->h_sc);
   const int st = batch_normalize(b, nullptr);  // members left in the batch
   for (hg_ctx *c : b->members) {  // ordinary contexts again
-    c->in_batch = false;
-    c->batch = nullptr;
-    lend_sets(c);
+    leave_batch(c);
   }
   if (b->d_bpar) hipFree(b->d_bpar);
   hipStreamDestroy(b->stream);
@@ -1756,9 +1763,7 @@ extern "C" int hg_batch_remove(hg_batch *b, hg_ctx *c) {
       if (st) return st;
       b->members.erase(b->members.begin() + q);
       b->sc_valid.erase(b->sc_valid.begin() + q);
-      c->in_batch = false;
-      c->batch = nullptr;
-      lend_sets(c);
+      leave_batch(c);
       // keep the cached member states aligned with the member list (the
       // array holds a record per member since hg_batch_add)
       for (size_t r = q; r < b->members.size(); ++r) b->h_sc[r] = b->h_sc[r + 1];

@@ -144,6 +144,7 @@ def test_gpu_separate_batch_gives_the_sets_back(hiplib, flow, separate, when):
         assert f0 - free() <= need + 0.1 * SETS
         b.remove(eng)
         b.close()
+        assert form(eng, N, own * 2)  # and takes its own form again
         out.append(fields(eng, flow))
         eng.close()
     same(out[0], out[1])
