@@ -113,6 +113,11 @@ static void lend_sets(hg_ctx *c) {
   const Use lock(l.mu);
   if (std::find(l.list.begin(), l.list.end(), c) == l.list.end()) l.list.push_back(c);
 }
+static bool any_lender() {
+  Lenders &l = lenders();
+  const Use lock(l.mu);
+  return !l.list.empty();
+}
 static int drop_sets(hg_ctx *c);
 
 // Frees one lender's sets on this device; false if there is none.
@@ -143,8 +148,8 @@ static int dev_malloc(size_t bytes, void **p) {
   // the queue.
   constexpr size_t RESERVE = 128 << 20;
   size_t left = 0, total = 0;
-  while (bytes >= 1 << 20 && hipMemGetInfo(&left, &total) == hipSuccess && left < RESERVE &&
-         take_back(device)) {
+  while (bytes >= 1 << 20 && any_lender() && hipMemGetInfo(&left, &total) == hipSuccess &&
+         left < RESERVE && take_back(device)) {
   }
   return HG_OK;
 }
@@ -1373,12 +1378,8 @@ static int ensure_fused_buffers(hg_ctx *c, int L, bool spare) {
   Dev &D = c->D;
   const size_t fb = sizeof(double) * (size_t)D.ncell;
   auto get = [&](size_t bytes, void **p) -> int {
-    size_t left = 0, total = 0;
     if (!spare) return dev_malloc(bytes, p);
-    if (hipMemGetInfo(&left, &total) == hipSuccess &&
-        left >= bytes + std::min(total / 8, 16 * bytes + ((size_t)256 << 20)) &&
-        hipMalloc(p, bytes) == hipSuccess)
-      return HG_OK;
+    if (hipMalloc(p, bytes) == hipSuccess) return HG_OK;
     (void)hipGetLastError();
     *p = nullptr;
     return HG_ERR_NOMEM;
@@ -1390,6 +1391,15 @@ static int ensure_fused_buffers(hg_ctx *c, int L, bool spare) {
       slot.push_back(&c->alt_W[w]);
       slot2.push_back(&c->alt2_W[w]);
     }
+  if (spare) {
+    const size_t want = field_pitch(fb) * (slot.size() + slot2.size());
+    size_t left = 0, total = 0;
+    if (hipMemGetInfo(&left, &total) != hipSuccess ||
+        left < want + std::min(total / 8, 16 * want + ((size_t)256 << 20))) {
+      (void)hipGetLastError();
+      return HG_ERR_NOMEM;
+    }
+  }
   void *m1 = nullptr, *m2 = nullptr, *part = nullptr;
   int st = HG_OK;
   if (!c->alt_ready) st = get(field_pitch(fb) * slot.size(), &m1);
